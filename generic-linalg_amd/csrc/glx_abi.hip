@@ -11,6 +11,7 @@
 // (verbosity.h:73-129).
 #include "../../include/glx.h"
 #include "glx_internal.h"
+#include "glx_resident.h"
 #include "glx_solvers.h"
 
 #include <algorithm>
@@ -1376,6 +1377,9 @@ int glx_set_tuning(int group, int use_graph) {
   });
 }
 
+int glx_set_resident(int on, int spins) {
+  return guarded([&] { set_resident(on, spins); });
+}
 int glx_set_sstep(int s, int rows) {
   return guarded([&] { set_sstep(s, rows); });
 }
@@ -1598,6 +1602,7 @@ int glx_autotune_normal(glx_lattice lat, int reps, int* rows64, int* rows32, dou
     so.eps = 0.0;
     so.group = g_group;
     so.use_graph = g_use_graph != 0;
+    so.per_launch = true;  // the shapes are those of the launch per iteration
     MixedOpts mo;
     mo.link_prec = LINKS_F32;
     mo.sstep = 1;  // the table shapes the one-iteration kernel; the s-step kernel has its own rows

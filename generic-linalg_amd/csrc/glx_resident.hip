@@ -1,0 +1,127 @@
+// glx_resident.hip -- the resident-system kernels' instances, launch shapes
+// and host-side bookkeeping (glx_resident.h).
+#include "glx_resident.h"
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <mutex>
+
+namespace glx {
+
+namespace {
+std::atomic<int> g_on{1};
+// a poll takes about a microsecond: a second in all before a wait gives up
+constexpr int kSpins = 1 << 20;
+std::atomic<int> g_spins{kSpins};
+
+constexpr int kMaxDevices = 64;
+int current_device() {
+  int d = 0;
+  GLX_HIP(hipGetDevice(&d));
+  if (d < 0 || d >= kMaxDevices) throw ArgError("device index beyond the resident-solve table");
+  return d;
+}
+int device_cus(int dev) {
+  static std::atomic<int> cus[kMaxDevices];
+  int n = cus[dev].load();
+  if (n == 0) {
+    GLX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+    cus[dev].store(n);
+  }
+  return n;
+}
+
+struct Slots {
+  std::mutex mu;
+  std::condition_variable cv;
+  int used[kMaxDevices] = {};
+};
+Slots& slots() {
+  static Slots* s = new Slots;  // outlives every static user
+  return *s;
+}
+
+__global__ __launch_bounds__(kBlock) void k_rs_fill(unsigned long long* q, long n, RsOut* out) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *out = RsOut{0, 0, 0, 0, 0.0, 0.0};
+  for (long i = long(blockIdx.x) * kBlock + threadIdx.x; i < n; i += long(gridDim.x) * kBlock) q[i] = kRsEmpty;
+}
+
+// rows per wave the kernels are instantiated for
+constexpr int kRows[] = {1, 2, 3, 4, 6, 8, 10};
+
+template <class T, int M>
+void launch(hipStream_t st, const RsGeom& g, const RsSolve& so) {
+  const long words = rs_exchange_words(g, rs_words<T>());
+  hipLaunchKernelGGL(k_rs_fill, dim3(unsigned(std::min<long>((words + kBlock - 1) / kBlock, 2048))), dim3(kBlock), 0,
+                     st, so.lines, words, so.out);
+  GLX_CHECK_LAUNCH();
+  const dim3 grid(g.nsx * g.nsy), block(kRsThreads);
+#define GLX_RS(R)                                                                              \
+  case R:                                                                                      \
+    hipLaunchKernelGGL((k_rs_cg<T, R, M>), grid, block, 0, st, g, so);             \
+    break;
+  switch (g.rows) {
+    GLX_RS(1)
+    GLX_RS(2)
+    GLX_RS(3)
+    GLX_RS(4)
+    GLX_RS(6)
+    GLX_RS(8)
+    GLX_RS(10)
+    default:
+      throw ArgError("no resident kernel for this tiling");
+  }
+#undef GLX_RS
+  GLX_CHECK_LAUNCH();
+}
+}  // namespace
+
+void set_resident(int on, int spins) {
+  g_on.store(on ? 1 : 0);
+  g_spins.store(spins > 0 ? spins : kSpins);
+}
+bool resident_on() { return g_on.load() != 0; }
+int resident_spins() { return g_spins.load(); }
+
+bool rs_plan(int lx, int ly, RsGeom& g) {
+  if (lx < 4 || long(lx) * ly > (1L << 24)) return false;
+  const int cap = std::min(kRsMaxBlocks, device_cus(current_device()));
+  const int nsx = (lx + kRsCols - 1) / kRsCols;
+  for (int r : kRows) {
+    if (ly < kRsWaves * r) break;  // a tile has this many rows
+    const int nsy = (ly + kRsWaves * r - 1) / (kRsWaves * r);
+    // few rows per wave only while that takes few blocks: the reductions
+    // grow with the blocks, the hops with the rows
+    const int most = r == 1 ? std::min(cap, 64) : (r == 2 ? std::min(cap, 128) : cap);
+    if (long(nsx) * nsy <= most) {
+      g = RsGeom{lx, ly, nsx, nsy, r};
+      return true;
+    }
+  }
+  return false;
+}
+
+void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so) {
+  if (mode == RS_REF) launch<c128, RS_REF>(st, g, so);
+  else if (mode == RS_ONE) launch<c128, RS_ONE>(st, g, so);
+  else launch<c64, RS_MIXED>(st, g, so);
+}
+
+RsReserve::RsReserve(int blocks) : dev_(current_device()), blocks_(blocks) {
+  const int cap = std::max(device_cus(dev_), blocks);
+  Slots& t = slots();
+  std::unique_lock<std::mutex> l(t.mu);
+  t.cv.wait(l, [&] { return t.used[dev_] + blocks_ <= cap; });
+  t.used[dev_] += blocks_;
+}
+RsReserve::~RsReserve() {
+  Slots& t = slots();
+  {
+    std::lock_guard<std::mutex> l(t.mu);
+    t.used[dev_] -= blocks_;
+  }
+  t.cv.notify_all();
+}
+
+}  // namespace glx

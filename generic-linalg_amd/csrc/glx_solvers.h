@@ -41,6 +41,7 @@ struct SolveOpts {
   int chunk = 16;           // iterations enqueued between convergence checks
   int group = 8;            // single-pass CG: iterations per enqueued group
   bool use_graph = true;    // single-pass CG: replay one captured hipGraph per group
+  bool per_launch = false;  // a launch per iteration also where the system would run resident (launch tuning)
 };
 
 // x (in: initial guess, out: solution) and b are device pointers of the

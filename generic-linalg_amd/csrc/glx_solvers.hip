@@ -13,6 +13,7 @@
 // zeta, ...) are computed on the device by the reduction finalisers and read
 // by the next kernel; the host reads the 16-byte control word once per chunk.
 #include "glx_solvers.h"
+#include "glx_resident.h"
 #include "glx_sstep.h"
 #include "glx_sswave.h"
 
@@ -22,6 +23,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <optional>
 
 namespace glx {
 
@@ -165,44 +167,6 @@ void DevicePool::trim() {
   if (!free_.empty()) (void)hipDeviceSynchronize();
   for (auto& kv : free_) (void)hipFree(kv.second);
   free_.clear();
-}
-
-// ========================================================= solver state ===
-constexpr int kMaxShift = 64;
-
-struct SolveState {
-  // control word (first 16 bytes, mirrored to the host)
-  int k, done, kfinal, n_rem;
-  int max_iter, resid_freq, worst_first, n_shift;
-  double eps, bsqrt, rsq, rsqNew;
-  double beta_r, resSq, maxrr, delta;  // maxrr: single-pass CG: max of |r|^2 since the last reliable update
-  int reliable, pending, ko;  // pending: self-finalising single-pass CG; ko: s-step CG launches
-  int n_xupd;  // multishift: shifts active before this iteration's check (their x still takes its update)
-  c128 alpha, alpha_prev, beta, beta_prev, rho, omega, pap;
-  double* hist;
-  double* resvec;
-  // host-mapped copy of `done` (single-pass CG): the kernels that change
-  // `done` also store it here, so the host polls it without a copy command
-  int* hdone;
-  // multishift
-  c128 zeta[kMaxShift], zeta_p[kMaxShift], alpha_s[kMaxShift], beta_s[kMaxShift];
-  double shifts[kMaxShift];
-  int mapping[kMaxShift];
-  int vec[kMaxShift];
-  // multishift: sums over the iterations of the shifts whose x_s (n_xupd)
-  // and p_s (n_rem after the check) were updated -- the pass's algorithmic
-  // bytes are 16 (3 upd_x + upd_p) per site
-  long long upd_x, upd_p;
-};
-
-struct Mirror {
-  int k, done, kfinal, n_rem;
-};
-
-template <class T>
-__device__ __forceinline__ typename Scal<T>::type as_scal(c128 a) {
-  if constexpr (is_cx<T>::value) return a;
-  else return a.re;
 }
 
 // Pinned slots for the control-word read-back (per host thread).
@@ -2501,6 +2465,79 @@ double time_sscg_traffic_impl(const DevOperator& o, int link_prec, int reps) {
   return double(ms) / reps;
 }
 
+// ===================================================== resident systems ===
+// CG on D^dag D (or the compact even/odd Schur operator) with the system held
+// on the chip (k_rs_cg, glx_resident.h).  A solve whose kernels gave up
+// waiting for each other (another process holding the chip) reports nothing
+// and leaves x a valid starting point: the caller then runs the solve with a
+// launch per iteration.
+static bool rs_fits(const DevOperator& o, RsGeom& g) {
+  if (!resident_on() || !o.tiled()) return false;
+  if (o.kind == OP_STAG_EO_SCHUR) {
+    // the sizes the compact operator is defined for (eo_fits)
+    if ((o.lx / 2) % 64 || o.ly % 4 || o.ly < 8) return false;
+  } else if (o.kind != OP_STAG_NORMAL) {
+    return false;
+  }
+  return rs_plan(o.lx, o.ly, g);
+}
+
+// One solve: FP64 in the reference's order (RS_REF) or single-pass (RS_ONE),
+// or mixed precision (RS_MIXED).
+static std::optional<SolveResult> rs_solve(const DevOperator& o, c128* x, const c128* b, const SolveOpts& opt,
+                                           RsMode mode, const MixedOpts& mo, const RsGeom& g) {
+  OwnedStream own(opt.stream);
+  hipStream_t st = own.st;
+  RsSolve so{};
+  so.x = x;
+  so.b = b;
+  so.u64 = o.u64;
+  so.lk = RsLinks{o.u64, nullptr, LINKS_F64};
+  if (mode == RS_MIXED)
+    so.lk = mo.link_prec == LINKS_F16 ? RsLinks{o.u16, o.sc16, LINKS_F16} : RsLinks{o.u32, nullptr, LINKS_F32};
+  if (!so.u64 || !so.lk.u || (so.lk.prec == LINKS_F16 && !so.lk.sc))
+    throw ArgError("operator has no links of this precision on the device");
+  so.mass = o.mass;
+  so.eps = opt.eps;
+  so.delta = mo.delta;
+  so.max_iter = opt.max_iter;
+  so.eo = o.kind == OP_STAG_EO_SCHUR ? 1 : 0;
+  so.spins = resident_spins();
+  DevBuf ex(size_t(rs_exchange_words(g, mode == RS_MIXED ? rs_words<c64>() : rs_words<c128>())) * 8);
+  DevBuf out(sizeof(RsOut)), hist(opt.want_hist ? size_t(opt.max_iter) * sizeof(double) : 0);
+  so.lines = ex.as<unsigned long long>();
+  so.ring = so.lines + long(kRsBufs) * kRsMaxBlocks * kRsLine;
+  so.out = out.as<RsOut>();
+  so.hist = hist.as<double>();
+  RsOut h{};
+  {
+    RsReserve slots(g.nsx * g.nsy);
+    rs_launch(st, g, mode, so);
+    GLX_HIP(hipMemcpyAsync(&h, so.out, sizeof(h), hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipStreamSynchronize(st));
+  }
+  if (h.err || !h.done) return std::nullopt;
+  SolveResult res;
+  res.name = mode == RS_REF ? "CG" : (mode == RS_ONE ? "CG-fused" : "CG-mixed");
+  res.iter = h.kfinal + 1;
+  res.resSq = h.resSq;
+  res.bsqrt = h.bsqrt;
+  res.reliable_updates = h.reliable;
+  if (mode == RS_MIXED) {
+    res.success = h.resSq == 0.0 || std::sqrt(h.resSq) < opt.eps * h.bsqrt;
+    res.ops_count = h.kfinal + 2 + h.reliable;
+  } else {
+    res.success = h.kfinal != opt.max_iter - 1;
+    res.ops_count = h.kfinal + 3;
+  }
+  if (opt.want_hist) {
+    res.relres_hist.resize(res.iter);
+    GLX_HIP(hipMemcpyAsync(res.relres_hist.data(), so.hist, sizeof(double) * res.iter, hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipStreamSynchronize(st));
+  }
+  return res;
+}
+
 // ============================================================ dispatch ====
 static bool real_op(const DevOperator& o) {
   return o.is_host() ? !o.host_complex : o.kind == OP_LAPLACE_REAL;
@@ -2508,6 +2545,9 @@ static bool real_op(const DevOperator& o) {
 
 SolveResult dev_cg(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
   if (real_op(op)) return cg_impl<double>(op, static_cast<double*>(x), static_cast<const double*>(b), o);
+  RsGeom g;
+  if (o.max_iter > 0 && rs_fits(op, g))
+    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_REF, MixedOpts{}, g)) return *r;
   return cg_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o);
 }
 SolveResult dev_bicgstab(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
@@ -2527,6 +2567,12 @@ SolveResult dev_cg_m(const DevOperator& op, void* const* xs, const void* b, int 
                          resid_freq_check, worst_first, o);
 }
 SolveResult dev_cg_mixed(const DevOperator& op, void* x, const void* b, const SolveOpts& o, const MixedOpts& m) {
+  // resident where the system fits, unless a launch form was asked for
+  RsGeom g;
+  if (o.max_iter > 0 && m.sstep == 0 && sstep_default() == 2 && sstep_rows() == 0 && sstep_form() < 0 &&
+      rs_fits(op, g)) {
+    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_MIXED, m, g)) return *r;
+  }
   if (!real_op(op) && (m.sstep ? m.sstep : sstep_default()) == 2 && sscg_fits(op)) {
     const int rows = sstep_rows_for(op.lx, op.ly);  // 0: the one-iteration form for this size
     if (rows > 0) return sscg_impl(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, m, rows);
@@ -2537,6 +2583,9 @@ SolveResult dev_cg_mixed(const DevOperator& op, void* x, const void* b, const So
 }
 SolveResult dev_cg_fused(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
   MixedOpts m;
+  RsGeom g;
+  if (o.max_iter > 0 && !o.per_launch && !real_op(op) && rs_fits(op, g))
+    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_ONE, m, g)) return *r;
   if (real_op(op))
     return fastcg_impl<double, double, false>(op, static_cast<double*>(x), static_cast<const double*>(b), o, m);
   return fastcg_impl<c128, c128, false>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, m);

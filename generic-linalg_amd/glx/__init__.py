@@ -208,6 +208,9 @@ def lib():
         L.glx_dev_cg_fused.argtypes = [vp, i, d, vp, vp, i, d, VP, IP]
         L.glx_set_tuning.restype = i
         L.glx_set_tuning.argtypes = [i, i]
+        if hasattr(L, "glx_set_resident"):  # absent from builds that predate it
+            L.glx_set_resident.restype = i
+            L.glx_set_resident.argtypes = [i, i]
         L.glx_set_sstep.restype = i
         L.glx_set_sstep.argtypes = [i, i]
         L.glx_get_sstep.restype = i
@@ -654,6 +657,13 @@ def staggered_grad(lat, mass: float, phi: DeviceArray, precision: int = 0, max_i
 
 def set_tuning(group: int = 16, use_graph: bool = False):
     _check(lib().glx_set_tuning(group, int(use_graph)), "glx_set_tuning")
+
+
+def set_resident(on: bool = True, spins: int = 0):
+    """Whether solves whose system fits the chip run in one launch (default),
+    and how often a block polls for another's value before the launch gives
+    up and the solve runs with a launch per iteration (0: the default)."""
+    _check(lib().glx_set_resident(int(on), int(spins)), "glx_set_resident")
 
 
 def set_sstep(s: int = 2, rows: int = 0):

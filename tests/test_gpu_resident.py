@@ -1,0 +1,177 @@
+"""Solves with the system held on the chip (glx_resident.h): CG on D^dag D in
+the reference's order, single-pass and mixed precision, and the even/odd
+solves, at the sizes where the tiling can go wrong -- strips of one column
+count and of two, 60 and 61 columns, bands whose last one shares rows with the
+band before it, every number of rows per wave, lattices of one tile, odd sizes
+-- and the way back to a launch per iteration when a wait runs out."""
+import threading
+
+import numpy as np
+import pytest
+
+from helpers import ENVELOPE, eo_envelope, lattice_inputs, relerr
+
+pytestmark = pytest.mark.gpu
+
+# lx, ly: 4 and 60 columns in one strip, 61 in two; ly = 8 one band, 9 a last
+# band sharing 7 rows; 512 to 1020 rows take 3 to 10 rows per wave with the
+# strips they have
+SIZES = [(4, 8), (5, 9), (60, 8), (61, 23), (64, 16), (130, 70), (97, 301), (330, 222)]
+LARGE = [(300, 512), (512, 400), (700, 512), (780, 780), (1000, 900)]
+
+
+@pytest.fixture
+def resident(glx):
+    yield glx.set_resident
+    glx.set_resident(True, 0)
+
+
+def system(glx, orc, lx, ly, beta=6.25):
+    links, b, _ = lattice_inputs(orc, lx, ly, beta=beta, seed=1000 + lx + 3 * ly)
+    return links, b, glx.Lattice(links, lx, ly), glx.DeviceArray(b)
+
+
+@pytest.mark.parametrize("lx,ly", SIZES)
+def test_cg_matches_oracle(glx, orc, lx, ly):
+    """Reference order: the iterations and ops_count of the oracle with its
+    serial or its correctly rounded sums (60 x 8: 125 and 124, 130 x 70: 178
+    and 177), x to the bound the staggered solver tests use; single-pass:
+    within 2 iterations."""
+    m = 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    kw = dict(links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-10)
+    runs = [orc.solve("cg", "staggered_normal", b, None, reductions=red, **kw) for red in ("serial", "extended")]
+    dx = glx.DeviceArray(np.zeros_like(b))
+    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+    assert ig.iter in [io.iter for _, io in runs]
+    xo, io = next(r for r in runs if r[1].iter == ig.iter)
+    assert (ig.ops_count, ig.success) == (io.ops_count, io.success)
+    assert relerr(dx.download(), xo) < 1e-11
+    dx.upload(np.zeros_like(b))
+    jg = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db, max_iter=5000)
+    assert abs(jg.iter - io.iter) <= 2 and jg.success
+    r = b - orc.apply("staggered_normal", dx.download(), links, m, lx, ly)
+    # (A x is rounded to 4 u |x|, and |x| <= |b| / m^2 = 100 |b|: 1e-13 |b|)
+    assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(b)
+    assert abs(np.sqrt(jg.resSq) - np.linalg.norm(r)) <= 1e-13 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("links_prec", [1, 2])
+@pytest.mark.parametrize("lx,ly", SIZES)
+def test_mixed_matches_oracle(glx, orc, lx, ly, links_prec):
+    m = 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    xs, _ = orc.solve("cg", "staggered_normal", b, None, links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-13)
+    dx = glx.DeviceArray(np.zeros_like(b))
+    info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, link_prec=links_prec)
+    x = dx.download()
+    r = b - orc.apply("staggered_normal", x, links, m, lx, ly)
+    assert info.success and info.reliable_updates > 0
+    assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(b)
+    # |x - x*| = |A^-1 r| <= |r| / m^2 (and x* is good to 1e-13 |b| / m^2)
+    assert np.linalg.norm(x - xs) <= 1.01e-10 * np.linalg.norm(b) / m**2
+
+
+@pytest.mark.parametrize("lx,ly", LARGE)
+def test_large_tiles_match_the_launch_per_iteration(glx, orc, resident, lx, ly):
+    """Both run the same algorithm; their solutions stop at the same residual
+    (1e-10 on a system of condition 1e3) within an iteration of each other."""
+    m = 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    out = {}
+    for on in (False, True):
+        resident(on)
+        for name in ("cg", "fused", "mixed"):
+            dx = glx.DeviceArray(np.zeros_like(b))
+            if name == "cg":
+                info = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db)
+            elif name == "fused":
+                info = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db)
+            else:
+                info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
+            assert info.success
+            out[name, on] = (info, dx.download())
+    for name in ("cg", "fused", "mixed"):
+        (i0, x0), (i1, x1) = out[name, False], out[name, True]
+        assert abs(i0.iter - i1.iter) <= (1 if name != "mixed" else max(6, 0.03 * i0.iter)), name
+        assert relerr(x1, x0) < 1e-10, name
+
+
+@pytest.mark.parametrize("lx,ly", [(128, 8), (256, 72), (384, 100)])
+@pytest.mark.parametrize("method", ["cg", "cg_fused", "mixed", "mixed_f16"])
+def test_even_odd(glx, orc, lx, ly, method):
+    m = 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    xs, err = eo_envelope(orc, b, links, m, lx, ly)
+    dx = glx.DeviceArray(np.zeros_like(b))
+    info, _ = glx.dev_solve_staggered_eo(lat, m, dx, db, method)
+    assert info.success
+    assert relerr(dx.download(), xs) <= ENVELOPE * err
+
+
+def test_guess_stop_and_zero(glx, orc):
+    """A guess that is nearly the solution, max_iter stops, b = 0."""
+    lx, ly, m = 130, 70, 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    kw = dict(links=links, mass=m, lx=lx, ly=ly)
+    x0, _ = orc.solve("cg", "staggered_normal", b, None, max_iter=5000, eps=1e-6, **kw)
+    xo, io = orc.solve("cg", "staggered_normal", b, x0, max_iter=5000, eps=1e-10, **kw)
+    dx = glx.DeviceArray(x0)
+    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+    # (nearest: the serial sums round differently)
+    assert abs(ig.iter - io.iter) <= 1 and relerr(dx.download(), xo) < 1e-9
+    for stop in (1, 2, 7):
+        xo, io = orc.solve("cg", "staggered_normal", b, None, max_iter=stop, eps=1e-10, **kw)
+        dx = glx.DeviceArray(np.zeros_like(b))
+        ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=stop)
+        assert (ig.iter, ig.success, ig.ops_count) == (io.iter, io.success, io.ops_count)
+        assert relerr(dx.download(), xo) < 1e-12 and abs(ig.resSq - io.resSq) < 1e-10 * io.resSq
+        dx.upload(np.zeros_like(b))
+        im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, max_iter=stop)
+        assert not im.success and im.iter == stop and relerr(dx.download(), xo) < 1e-4
+    z = glx.DeviceArray(np.zeros_like(b))
+    dx = glx.DeviceArray(np.zeros_like(b))
+    im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, z)
+    assert im.success and im.resSq == 0.0 and not dx.download().any()
+
+
+def test_waits_that_run_out(glx, orc, resident):
+    """With a single poll per wait the launch gives up, and the solve runs with
+    a launch per iteration: the same answer."""
+    lx, ly, m = 130, 70, 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    xo, io = orc.solve("cg", "staggered_normal", b, None, links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-10)
+    resident(True, 1)
+    dx = glx.DeviceArray(np.zeros_like(b))
+    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+    assert abs(ig.iter - io.iter) <= 1 and relerr(dx.download(), xo) < 1e-9
+    dx.upload(np.zeros_like(b))
+    assert glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db).success
+    assert relerr(dx.download(), xo) < 1e-9
+
+
+def test_threads_share_the_chip(glx, orc):
+    """Solves from several host threads at once, together wanting more blocks
+    than there are CUs, give the bits each gives alone."""
+    m = 0.1
+    work = [system(glx, orc, lx, ly) for lx, ly in ((700, 512), (330, 222), (512, 400), (256, 256))]
+    alone, got = [], [None] * len(work)
+    for _, b, lat, db in work:
+        dx = glx.DeviceArray(np.zeros_like(b))
+        glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
+        alone.append(dx.download())
+
+    def run(k):
+        _, b, lat, db = work[k]
+        for _ in range(3):
+            dx = glx.DeviceArray(np.zeros_like(b))
+            glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
+            got[k] = dx.download()
+
+    ts = [threading.Thread(target=run, args=(k,)) for k in range(len(work))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for a, g in zip(alone, got):
+        assert np.array_equal(a, g)
