@@ -40,6 +40,18 @@
 // measured 1.9 us for 256 blocks and one sum, 2.2 us for four sums; eight
 // blocks per line 2.9 and 7.8 us.
 //
+// Ring slots: boundary rows lie by lattice site (whole rows, coalesced);
+// boundary columns by block and row, four values side by side, so that a wave
+// stores them in whole lines.  With the columns by lattice site as well (two
+// 16-byte pieces per row) 1024^2 took 6.97 us per iteration in mixed
+// precision and 13.2 us in FP64, against 6.1 and 10.6 us.
+//
+// Measured (us per iteration: reference order, single-pass FP64, mixed):
+// 64^2 4.3, 2.9, 3.2; 256^2 5.3, 3.6, 3.6; 512^2 6.8, 4.6, 4.4; 1024^2 10.6,
+// 10.4, 6.1.  A launch per iteration took 17, 12, 14; 18, 12, 10; 21, 13, 10;
+// 38, 30, 14.  (Of an iteration at 256^2, 1.3 us is the round trip of the
+// reduction, the rest the latencies of the hops, LDS and block sums.)
+//
 // Every wait is bounded (RsSolve::spins polls): a block that gives up sets the
 // error word and leaves; the others run out of polls as well, nothing of the
 // result is used, and the host repeats the solve with a launch per iteration.
@@ -93,7 +105,7 @@ struct RsSolve {
   int eo;          // compact even-site vectors
   int spins;       // polls per wait
   double* hist;    // iterated relative residual per iteration, or null
-  unsigned long long* ring;   // [kRsBufs][lx * ly][64-bit words of T]
+  unsigned long long* ring;   // [kRsBufs][lx * ly] rows by lattice site, then [kRsBufs][blocks][8 R][4] columns, of T
   unsigned long long* lines;  // [kRsBufs][kRsMaxBlocks][kRsLine]
   RsOut* out;
 };
@@ -301,11 +313,17 @@ enum RsHaloVal : int { RS_RH = 0, RS_PH = 2, RS_APH = 4, RS_UXH = 6, RS_UYH, RS_
 template <class T, int R>
 struct RsShared {
   static constexpr bool kX = sizeof(T) == 16 && R >= 4;
-  T v[2][kRsWaves][2][64];
+  // the largest FP64 tile keeps four rows of r and U_y above the run here as
+  // well, and p and q share one buffer (with a barrier of their own)
+  static constexpr int kR = sizeof(T) == 16 && R > 8 ? 4 : 0;
+  static constexpr int kV = kR ? 1 : 2;
+  T v[kV][kRsWaves][2][64];
   T rim[kRsWaves][R][4];  // the run's two columns each side: published, then the neighbours'
   double part[kRsWaves][4], tot[kRsWaves][4];
   int bad;
   T x[kX ? R : 1][kX ? kRsThreads : 1];
+  T r[kR ? kR : 1][kR ? kRsThreads : 1];
+  T uyt[kR ? kRsThreads : 1];
   T h[kX ? 2 : 1][RS_NHALO][kX ? 64 : 1];
 };
 
@@ -339,8 +357,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     return y < 0 ? y + ly : y;
   };
   // a vector's entry at (xg, y), or -1 where a compact vector has none
-  // (the column passes through an empty asm here and in slot(), so that the
-  // compiler does not keep the addresses of every row in registers)
+  // (rows and columns pass through empty asm statements here and below, so
+  // that the compiler does not keep the addresses of every row in registers)
   auto at = [&](int y) -> int {
     int x = xg;
     asm volatile("" : "+v"(x));
@@ -356,16 +374,22 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
   }
   pub = __builtin_amdgcn_readfirstlane(pub);
 
-  T r[R], p[R], ap[R], ux[R], uy[R], xr[Sh::kX ? 1 : R], uxm[sizeof(T) == 8 ? R : 1];
+  T rv_[R - Sh::kR], p[R], ap[R], ux[R], uy[R], xr[Sh::kX ? 1 : R], uxm[sizeof(T) == 8 ? R : 1];
   auto xref = [&](int j) -> T& {
     if constexpr (Sh::kX) return sh.x[j][threadIdx.x];
     else return xr[j];
+  };
+  auto rref = [&](int j) -> T& {
+    if constexpr (Sh::kR != 0) {
+      if (j >= R - Sh::kR) return sh.r[j - (R - Sh::kR)][threadIdx.x];
+    }
+    return rv_[j < R - Sh::kR ? j : 0];
   };
   auto uxm_of = [&](int j) -> T { return uxm[sizeof(T) == 8 ? j : 0]; };
   uxm[0] = zero_of<T>();
 #pragma unroll
   for (int j = 0; j < R; j++) {
-    r[j] = p[j] = ap[j] = ux[j] = uy[j] = zero_of<T>();
+    rref(j) = p[j] = ap[j] = ux[j] = uy[j] = zero_of<T>();
     T x = zero_of<T>();
     if (valid) {
       rs_links<Re>(so.lk, (yw + j) * lx + xg, ey, ux[j], uy[j]);
@@ -380,22 +404,27 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
   // U_y of the row above the run; on the edge waves the two rows beyond the
   // tile, nearest first (y0 - 1, y0 - 2 or y0 + L, y0 + L + 1), and the
   // nearest one's links with U_y of the row below it
-  T uyt = zero_of<T>(), hreg[Sh::kX ? 1 : RS_NHALO];
+  T uyt_reg = zero_of<T>(), hreg[Sh::kX ? 1 : RS_NHALO];
   auto hal = [&](int v) -> T& {  // (edge waves only)
     if constexpr (Sh::kX) return sh.h[top ? 0 : 1][v][lane];
     else return hreg[v];
   };
+  auto uyt = [&]() -> T& {
+    if constexpr (Sh::kR != 0) return sh.uyt[threadIdx.x];
+    else return uyt_reg;
+  };
   const int yh[2] = {wrapy(top ? y0 - 1 : y0 + L), wrapy(top ? y0 - 2 : y0 + L + 1)};
   {
-    T a, b = zero_of<T>(), ux0 = b, uy0 = b, uy1 = b;
+    T a, b = zero_of<T>(), ux0 = b, uy0 = b, uy1 = b, uyw = b;
     if (valid) {
-      rs_links<Re>(so.lk, wrapy(yw - 1) * lx + xg, ey, a, uyt);
+      rs_links<Re>(so.lk, wrapy(yw - 1) * lx + xg, ey, a, uyw);
       if (edge) {
         rs_links<Re>(so.lk, yh[0] * lx + xg, ey, ux0, uy0);
         rs_links<Re>(so.lk, yh[1] * lx + xg, ey, a, uy1);
         if (!top) uy1 = uy[R - 1];
       }
     }
+    uyt() = uyw;
     if (edge || !Sh::kX) {
 #pragma unroll
       for (int v = 0; v < RS_UXH; v++) hal(v) = b;
@@ -408,33 +437,38 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
 
   // ring slots: 32-bit byte offsets from the uniform base
   const unsigned row_bytes = unsigned(lx) * sizeof(T), buf_bytes = unsigned(ly) * row_bytes;
-  auto word = [&](int use, unsigned off) {
-    return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(so.ring) + (unsigned(use & 3) * buf_bytes + off));
-  };
   auto slot = [&](int use, int y) {
     unsigned off = unsigned(xg) * sizeof(T);
     asm volatile("" : "+v"(off));
-    return word(use, off + unsigned(y) * row_bytes);
+    off += unsigned(use & 3) * buf_bytes + unsigned(y) * row_bytes;
+    return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(so.ring) + off);
   };
   // The columns neighbours exchange pass through LDS, so that each of the 4 R
-  // values is one lane's: lane l moves row l / 4, the run's columns 0, 1, w - 2,
-  // w - 1 (published) and -2, -1, w, w + 1 (collected) for l % 4 = 0 .. 3.
+  // values of a run is one lane's: lane l moves row l / 4, the run's columns 0,
+  // 1, w - 2, w - 1 (published) and -2, -1, w, w + 1 (collected) for l % 4 =
+  // 0 .. 3.  Their slots lie by block and row, four in a row, so that a wave
+  // stores whole lines.
   const int mrow = lane >> 2, mcol = lane & 3;
   const bool mover = lane < 4 * R;
-  auto xoff = [&](int x) {  // ring offset of this lane's row in column x0 + x
-    x = (x0 + x) % lx;
-    return unsigned(x < 0 ? x + lx : x) * unsigned(sizeof(T)) + unsigned(yw + mrow) * row_bytes;
+  const unsigned col_bytes = unsigned(nblk) * unsigned(L * 4 * sizeof(T));
+  char* cols_base = reinterpret_cast<char*>(so.ring) + size_t(kRsBufs) * buf_bytes;
+  auto col_word = [&](int use, unsigned off) {
+    return reinterpret_cast<unsigned long long*>(cols_base + (unsigned(use & 3) * col_bytes + off));
   };
-  const unsigned put_off = mover ? xoff(mcol < 2 ? mcol : cols - 4 + mcol) : 0;
-  const unsigned get_off = mover ? xoff(mcol < 2 ? mcol - 2 : cols - 2 + mcol) : 0;
+  auto col_off = [&](int blk, int c) { return unsigned((blk * L + wave * R + mrow) * 4 + c) * unsigned(sizeof(T)); };
+  const int row0 = blockIdx.x - sx;  // the band's first block
+  const int left = row0 + (sx == 0 ? g.nsx - 1 : sx - 1), right = row0 + (sx == g.nsx - 1 ? 0 : sx + 1);
+  const unsigned put_off = col_off(blockIdx.x, mcol), get_off = col_off(mcol < 2 ? left : right, mcol ^ 2);
   const int scol = lane < 2 * kRsHalo ? lane - 2 : lane - cols + 2;  // a side lane's column of the four
   const int rcol = lane < kRsHalo ? lane : lane - cols;              // a rim lane's
   // f(slot, j) for the rows of the wave that other bands read
   auto for_rows = [&](int use, auto f) {
+    if (pub == 0) return;
+    if (own) {
 #pragma unroll
-    for (int j = 0; j < R; j++)
-      if (pub >> j & 1)
-        if (own && !side) f(slot(use, yw + j), j);
+      for (int j = 0; j < R; j++)
+        if (pub >> j & 1) f(slot(use, yw + j), j);
+    }
   };
   auto wave_fence = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -449,10 +483,10 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     }
     wave_fence();
     rs_stores_done();  // (the slots emptied since the last reduction)
-    if (mover) rs_put<T>(word(e, put_off), sh.rim[wave][mrow][mcol]);
+    if (mover) rs_put<T>(col_word(e, put_off), sh.rim[wave][mrow][mcol]);
     for_rows(e, [&](unsigned long long* q, int j) { rs_put<T>(q, v[j]); });
     rs_publish(sums, sh.part, so.lines, c);
-    if (mover) rs_empty<T>(word(e + 2, put_off));
+    if (mover) rs_empty<T>(col_word(e + 2, put_off));
     for_rows(e + 2, [&](unsigned long long* q, int) { rs_empty<T>(q); });
   };
   // Collects ring use e into the halo lanes of v and the halo rows hal(h) (RING),
@@ -463,7 +497,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     constexpr int J = (kRsMaxBlocks * ND + kRsThreads - 1) / kRsThreads;
     const int l0 = threadIdx.x / ND;
     const unsigned long long* base = so.lines + (c & 3) * kRsMaxBlocks * kRsLine + (lane & (ND - 1));
-    const bool need = l0 < nblk, far = edge && valid;
+    const bool need = l0 < nblk;
     unsigned long long q[J];
 #pragma unroll
     for (int i = 0; i < J; i++) q[i] = 0;
@@ -476,15 +510,15 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
 #pragma unroll
         for (int i = 0; i < J; i++) {
           const int b = l0 + i * (kRsThreads / ND);
-          if (b < nblk) q[i] = rs_load(base + b * kRsLine);
+          if (i == 0 || b < nblk) q[i] = rs_load(base + b * kRsLine);
         }
       }
       if constexpr (RING) {
-        if (far) {
+        if (edge && valid) {
           h0 = rs_read<T>(slot(e, yh[0]));
           h1 = rs_read<T>(slot(e, yh[1]));
         }
-        if (mover) m = rs_read<T>(word(e, get_off));
+        if (mover) m = rs_read<T>(col_word(e, get_off));
       }
       ok = true;
 #pragma unroll
@@ -569,7 +603,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
           cvt(dr, d);
 #pragma unroll
           for (int jj = 0; jj < R; jj++)
-            if (jj == j) r[jj] = dr;
+            if (jj == j) ap[jj] = dr;
         }
         qa = qb;
         qb = qc;
@@ -581,8 +615,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
         u1x = ucx;
         u1y = ucy;
       }
-      publish(r, e, s2, c);
-      if (!collect(with_ring, r, RS_RH, e, s2, c)) return give_up();
+      publish(ap, e, s2, c);
+      if (!collect(with_ring, ap, RS_RH, e, s2, c)) return give_up();
       e++;
       c++;
       if (first) {
@@ -601,7 +635,10 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
         k++;
       }
 #pragma unroll
-      for (int j = 0; j < R; j++) ap[j] = zero_of<T>();
+      for (int j = 0; j < R; j++) {
+        rref(j) = ap[j];
+        ap[j] = zero_of<T>();
+      }
       if (edge) hal(RS_APH) = hal(RS_APH + 1) = zero_of<T>();
     }
 
@@ -611,9 +648,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     for (int j = 0; j < R; j++) {
       if constexpr (M != RS_REF) {
         xref(j) = rs_axpy(a, p[j], xref(j));
-        r[j] = rs_axpy(-a, ap[j], r[j]);
+        rref(j) = rs_axpy(-a, ap[j], rref(j));
       }
-      p[j] = rs_axpy(be, p[j], r[j]);
+      p[j] = rs_axpy(be, p[j], rref(j));
     }
     if (edge) {
 #pragma unroll
@@ -642,13 +679,14 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     for (int j = 0; j < R; j++) {
       if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
       ap[j] = rs_hop(p[j], j ? p[j ? j - 1 : 0] : up, j + 1 < R ? p[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j),
-                     uy[j], j ? uy[j ? j - 1 : 0] : uyt);
+                     uy[j], j ? uy[j ? j - 1 : 0] : uyt());
     }
-    sh.v[1][wave][0][lane] = ap[0];
-    sh.v[1][wave][1][lane] = ap[R - 1];
+    if constexpr (Sh::kV == 1) __syncthreads();
+    sh.v[Sh::kV - 1][wave][0][lane] = ap[0];
+    sh.v[Sh::kV - 1][wave][1][lane] = ap[R - 1];
     __syncthreads();
-    up = top ? qh : sh.v[1][top ? 0 : wave - 1][1][lane];
-    below = wave == NW - 1 ? qh : sh.v[1][wave + 1 < NW ? wave + 1 : wave][0][lane];
+    up = top ? qh : sh.v[Sh::kV - 1][top ? 0 : wave - 1][1][lane];
+    below = wave == NW - 1 ? qh : sh.v[Sh::kV - 1][wave + 1 < NW ? wave + 1 : wave][0][lane];
     constexpr int N1 = M == RS_REF ? 2 : 4;
     double v1[N1];
 #pragma unroll
@@ -658,7 +696,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
       if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
       const T q = ap[j];
       const T v = rs_mhop(m2, p[j], q, up, j + 1 < R ? ap[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j), uy[j],
-                          j ? uy[j ? j - 1 : 0] : uyt);
+                          j ? uy[j ? j - 1 : 0] : uyt());
       up = q;
       ap[j] = v;
       if (wave * R + j >= shared) {
@@ -667,7 +705,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
         if constexpr (M == RS_REF) {
           v1[1] = __builtin_fma(pr, ai, __builtin_fma(-pi, ar, v1[1]));
         } else {
-          const double rr = r[j].re, ri = r[j].im;
+          const T rv = rref(j);
+          const double rr = rv.re, ri = rv.im;
           v1[1] = __builtin_fma(ar, ar, __builtin_fma(ai, ai, v1[1]));
           v1[2] = __builtin_fma(ar, rr, __builtin_fma(ai, ri, v1[2]));
           v1[3] = __builtin_fma(rr, rr, __builtin_fma(ri, ri, v1[3]));
@@ -690,8 +729,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
       double v2[1] = {0.0};
 #pragma unroll
       for (int j = 0; j < R; j++) {
-        r[j] = rs_axpy(ma, ap[j], r[j]);
-        if (wave * R + j >= shared) v2[0] = __builtin_fma(r[j].re, r[j].re, __builtin_fma(r[j].im, r[j].im, v2[0]));
+        const T rv = rs_axpy(ma, ap[j], rref(j));
+        rref(j) = rv;
+        if (wave * R + j >= shared) v2[0] = __builtin_fma(rv.re, rv.re, __builtin_fma(rv.im, rv.im, v2[0]));
       }
       v2[0] = own ? v2[0] : 0.0;
       rs_stores_done();  // (slots and lines emptied since the last reduction)
@@ -732,7 +772,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
 #pragma unroll
     for (int j = 0; j < R; j++) {
       if constexpr (M != RS_REF) xref(j) = rs_axpy(a, p[j], xref(j));
-      const int i = at(yw + j);
+      int y = yw;
+      asm volatile("" : "+s"(y));
+      const int i = at(y + j);
       if (own && i >= 0 && wave * R + j >= shared) {
         unsigned long long* q = reinterpret_cast<unsigned long long*>(so.x + i);
         c128 v;
@@ -771,7 +813,8 @@ bool rs_plan(int lx, int ly, RsGeom& g);
 // Words of the exchange buffers (lines, then ring) of a solve with `words`
 // 64-bit words per element.
 inline long rs_exchange_words(const RsGeom& g, int words) {
-  return long(kRsBufs) * (kRsMaxBlocks * kRsLine + long(g.lx) * g.ly * words);
+  const long columns = long(g.nsx) * g.nsy * kRsWaves * g.rows * 4;
+  return long(kRsBufs) * (kRsMaxBlocks * kRsLine + (long(g.lx) * g.ly + columns) * words);
 }
 // Empties the exchange buffers and clears the result record, then launches.
 void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so);

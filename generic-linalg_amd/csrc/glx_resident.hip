@@ -92,8 +92,14 @@ bool rs_plan(int lx, int ly, RsGeom& g) {
     if (ly < kRsWaves * r) break;  // a tile has this many rows
     const int nsy = (ly + kRsWaves * r - 1) / (kRsWaves * r);
     // few rows per wave only while that takes few blocks: the reductions
-    // grow with the blocks, the hops with the rows
-    const int most = r == 1 ? std::min(cap, 64) : (r == 2 ? std::min(cap, 128) : cap);
+    // grow with the blocks, the hops with the rows (us per iteration in the
+    // reference's order and mixed: 128^2 5.2 and 3.7 at 1 or 2 rows, 5.4 and
+    // 4.0 at 4; 256^2 6.2 and 4.1 at 1 row and 160 blocks, 5.9 and 3.9 at 2
+    // and 80, 5.9 and 4.4 at 4 and 40; 512^2 7.5 and 4.9 at 3 rows and 198
+    // blocks, 7.0 and 4.7 at 4 and 144, 7.4 and 5.2 at 6 and 99; 700^2 8.0 and
+    // 5.6 at 6 rows and 180 blocks, 8.6 and 5.8 at 8 and 132)
+    const int few = r == 1 ? 64 : (r == 2 ? 128 : (r == 3 ? 160 : kRsMaxBlocks));
+    const int most = std::min(cap, few);
     if (long(nsx) * nsy <= most) {
       g = RsGeom{lx, ly, nsx, nsy, r};
       return true;
