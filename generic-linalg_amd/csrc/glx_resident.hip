@@ -47,15 +47,21 @@ __global__ __launch_bounds__(kBlock) void k_rs_fill(unsigned long long* q, long 
   for (long i = long(blockIdx.x) * kBlock + threadIdx.x; i < n; i += long(gridDim.x) * kBlock) q[i] = kRsEmpty;
 }
 
+}  // namespace
+
+void rs_fill(hipStream_t st, const RsSolve& so, long words) {
+  hipLaunchKernelGGL(k_rs_fill, dim3(unsigned(std::min<long>((words + kBlock - 1) / kBlock, 2048))), dim3(kBlock), 0,
+                     st, so.lines, words, so.out);
+  GLX_CHECK_LAUNCH();
+}
+
+namespace {
 // rows per wave the kernels are instantiated for
 constexpr int kRows[] = {1, 2, 3, 4, 6, 8, 10};
 
 template <class T, int M>
 void launch(hipStream_t st, const RsGeom& g, const RsSolve& so) {
-  const long words = rs_exchange_words(g, rs_words<T>());
-  hipLaunchKernelGGL(k_rs_fill, dim3(unsigned(std::min<long>((words + kBlock - 1) / kBlock, 2048))), dim3(kBlock), 0,
-                     st, so.lines, words, so.out);
-  GLX_CHECK_LAUNCH();
+  rs_fill(st, so, rs_exchange_words(g, rs_words<T>(), 2));
   const dim3 grid(g.nsx * g.nsy), block(kRsThreads);
 #define GLX_RS(R)                                                                              \
   case R:                                                                                      \
@@ -84,11 +90,12 @@ void set_resident(int on, int spins) {
 bool resident_on() { return g_on.load() != 0; }
 int resident_spins() { return g_spins.load(); }
 
-bool rs_plan(int lx, int ly, RsGeom& g) {
-  if (lx < 4 || long(lx) * ly > (1L << 24)) return false;
+bool rs_plan(int lx, int ly, int halo, int most_rows, RsGeom& g) {
+  if (lx < 2 * halo || long(lx) * ly > (1L << 24)) return false;
   const int cap = std::min(kRsMaxBlocks, device_cus(current_device()));
-  const int nsx = (lx + kRsCols - 1) / kRsCols;
+  const int nsx = (lx + rs_cols(halo) - 1) / rs_cols(halo);
   for (int r : kRows) {
+    if (r > most_rows) break;
     if (ly < kRsWaves * r) break;  // a tile has this many rows
     const int nsy = (ly + kRsWaves * r - 1) / (kRsWaves * r);
     // few rows per wave only while that takes few blocks: the reductions

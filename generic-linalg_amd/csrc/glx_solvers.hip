@@ -2466,36 +2466,59 @@ double time_sscg_traffic_impl(const DevOperator& o, int link_prec, int reps) {
 }
 
 // ===================================================== resident systems ===
-// CG on D^dag D (or the compact even/odd Schur operator) with the system held
-// on the chip (k_rs_cg, glx_resident.h).  A solve whose kernels gave up
-// waiting for each other (another process holding the chip) reports nothing
-// and leaves x a valid starting point: the caller then runs the solve with a
-// launch per iteration.
-static bool rs_fits(const DevOperator& o, RsGeom& g) {
+// Solves with the system held on the chip (glx_resident.h, glx_reshop.h).  One
+// whose kernels gave up waiting for each other (another process holding the
+// chip) reports nothing and leaves x a valid starting point: the caller then
+// runs the solve with a launch per iteration.
+
+// A solver's resident form: which kernel and what it is called.
+enum RsForm : int { RSF_CG, RSF_FUSED, RSF_MIXED, RSF_BICGSTAB };
+
+// Whether the operator and its lattice have that form here.
+static bool rs_fits(const DevOperator& o, RsForm form, RsGeom& g) {
   if (!resident_on() || !o.tiled()) return false;
-  if (o.kind == OP_STAG_EO_SCHUR) {
-    // the sizes the compact operator is defined for (eo_fits)
-    if ((o.lx / 2) % 64 || o.ly % 4 || o.ly < 8) return false;
-  } else if (o.kind != OP_STAG_NORMAL) {
-    return false;
+  switch (o.kind) {
+    case OP_STAG_NORMAL:
+      return form != RSF_BICGSTAB && rs_plan(o.lx, o.ly, 2, kRsMostRows, g);
+    case OP_STAG_EO_SCHUR:
+      // the sizes the compact operator is defined for (eo_fits)
+      return form != RSF_BICGSTAB && (o.lx / 2) % 64 == 0 && o.ly % 4 == 0 && o.ly >= 8 &&
+             rs_plan(o.lx, o.ly, 2, kRsMostRows, g);
+    case OP_LAPLACE_REAL:
+      return form == RSF_CG && rs_plan(o.lx, o.ly, 1, kRsMostRowsHop, g);
+    case OP_LAPLACE:
+    case OP_LAPLACE_U1:
+      return (form == RSF_CG && rs_plan(o.lx, o.ly, 1, kRsMostRowsHop, g)) ||
+             (form == RSF_BICGSTAB && rs_plan(o.lx, o.ly, 1, kRsMostRowsBicg, g));
+    case OP_STAG:
+    case OP_STAG_DAG:
+      return form == RSF_BICGSTAB && rs_plan(o.lx, o.ly, 1, kRsMostRowsBicg, g);
+    default:
+      return false;
   }
-  return rs_plan(o.lx, o.ly, g);
 }
 
-// One solve: FP64 in the reference's order (RS_REF) or single-pass (RS_ONE),
-// or mixed precision (RS_MIXED).
-static std::optional<SolveResult> rs_solve(const DevOperator& o, c128* x, const c128* b, const SolveOpts& opt,
-                                           RsMode mode, const MixedOpts& mo, const RsGeom& g) {
-  OwnedStream own(opt.stream);
-  hipStream_t st = own.st;
+static std::optional<SolveResult> rs_solve(const DevOperator& o, void* x, const void* b, const SolveOpts& opt,
+                                           RsForm form, const MixedOpts& mo) {
+  RsGeom g;
+  if (opt.max_iter <= 0 || opt.per_launch || !rs_fits(o, form, g)) return std::nullopt;
+  // the stream these solvers run on: the reference-order ones the caller's
+  // (the null stream), the others one of their own
+  std::optional<OwnedStream> own;
+  hipStream_t st = opt.stream;
+  if (form == RSF_FUSED || form == RSF_MIXED) {
+    own.emplace(opt.stream);
+    st = own->st;
+  }
+  const bool cplx = o.kind != OP_LAPLACE_REAL, hop = o.kind != OP_STAG_NORMAL && o.kind != OP_STAG_EO_SCHUR;
   RsSolve so{};
-  so.x = x;
-  so.b = b;
+  so.x = static_cast<c128*>(x);
+  so.b = static_cast<const c128*>(b);
   so.u64 = o.u64;
   so.lk = RsLinks{o.u64, nullptr, LINKS_F64};
-  if (mode == RS_MIXED)
+  if (form == RSF_MIXED)
     so.lk = mo.link_prec == LINKS_F16 ? RsLinks{o.u16, o.sc16, LINKS_F16} : RsLinks{o.u32, nullptr, LINKS_F32};
-  if (!so.u64 || !so.lk.u || (so.lk.prec == LINKS_F16 && !so.lk.sc))
+  if (op_links(o.kind) && (!so.u64 || !so.lk.u || (so.lk.prec == LINKS_F16 && !so.lk.sc)))
     throw ArgError("operator has no links of this precision on the device");
   so.mass = o.mass;
   so.eps = opt.eps;
@@ -2503,7 +2526,16 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, c128* x, const 
   so.max_iter = opt.max_iter;
   so.eo = o.kind == OP_STAG_EO_SCHUR ? 1 : 0;
   so.spins = resident_spins();
-  DevBuf ex(size_t(rs_exchange_words(g, mode == RS_MIXED ? rs_words<c64>() : rs_words<c128>())) * 8);
+  if (o.kind == OP_STAG || o.kind == OP_STAG_DAG) {
+    so.diag = o.mass;
+    so.fx = o.kind == OP_STAG ? -0.5 : 0.5;
+    so.fy_odd = -so.fx;
+  } else {
+    so.diag = 4.0 + o.mass;
+    so.fx = so.fy_odd = -1.0;
+  }
+  const int words = cplx && form != RSF_MIXED ? rs_words<c128>() : 1;
+  DevBuf ex(size_t(rs_exchange_words(g, words, hop ? 1 : 2)) * 8);
   DevBuf out(sizeof(RsOut)), hist(opt.want_hist ? size_t(opt.max_iter) * sizeof(double) : 0);
   so.lines = ex.as<unsigned long long>();
   so.ring = so.lines + long(kRsBufs) * kRsMaxBlocks * kRsLine;
@@ -2512,23 +2544,36 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, c128* x, const 
   RsOut h{};
   {
     RsReserve slots(g.nsx * g.nsy);
-    rs_launch(st, g, mode, so);
+    if (form == RSF_BICGSTAB) rs_launch_hop_bicgstab(st, g, o.kind == OP_STAG || o.kind == OP_STAG_DAG ? -1 : 1, so);
+    else if (hop) rs_launch_hop_cg(st, g, cplx, so);
+    else rs_launch(st, g, form == RSF_CG ? RS_REF : (form == RSF_FUSED ? RS_ONE : RS_MIXED), so);
     GLX_HIP(hipMemcpyAsync(&h, so.out, sizeof(h), hipMemcpyDeviceToHost, st));
     GLX_HIP(hipStreamSynchronize(st));
   }
   if (h.err || !h.done) return std::nullopt;
   SolveResult res;
-  res.name = mode == RS_REF ? "CG" : (mode == RS_ONE ? "CG-fused" : "CG-mixed");
   res.iter = h.kfinal + 1;
   res.resSq = h.resSq;
   res.bsqrt = h.bsqrt;
   res.reliable_updates = h.reliable;
-  if (mode == RS_MIXED) {
-    res.success = h.resSq == 0.0 || std::sqrt(h.resSq) < opt.eps * h.bsqrt;
-    res.ops_count = h.kfinal + 2 + h.reliable;
-  } else {
-    res.success = h.kfinal != opt.max_iter - 1;
-    res.ops_count = h.kfinal + 3;
+  res.success = h.kfinal != opt.max_iter - 1;
+  res.ops_count = res.iter + 2;
+  switch (form) {
+    case RSF_CG:
+      res.name = "CG";
+      break;
+    case RSF_FUSED:
+      res.name = "CG-fused";
+      break;
+    case RSF_BICGSTAB:
+      res.name = "BiCGStab";
+      res.ops_count = 2 * res.iter + 2;
+      break;
+    case RSF_MIXED:
+      res.name = "CG-mixed";
+      res.success = h.resSq == 0.0 || std::sqrt(h.resSq) < opt.eps * h.bsqrt;
+      res.ops_count = h.kfinal + 2 + h.reliable;
+      break;
   }
   if (opt.want_hist) {
     res.relres_hist.resize(res.iter);
@@ -2544,13 +2589,12 @@ static bool real_op(const DevOperator& o) {
 }
 
 SolveResult dev_cg(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
+  if (auto r = rs_solve(op, x, b, o, RSF_CG, MixedOpts{})) return *r;
   if (real_op(op)) return cg_impl<double>(op, static_cast<double*>(x), static_cast<const double*>(b), o);
-  RsGeom g;
-  if (o.max_iter > 0 && rs_fits(op, g))
-    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_REF, MixedOpts{}, g)) return *r;
   return cg_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o);
 }
 SolveResult dev_bicgstab(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
+  if (auto r = rs_solve(op, x, b, o, RSF_BICGSTAB, MixedOpts{})) return *r;
   if (real_op(op)) return bicgstab_impl<double>(op, static_cast<double*>(x), static_cast<const double*>(b), o);
   return bicgstab_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o);
 }
@@ -2568,11 +2612,8 @@ SolveResult dev_cg_m(const DevOperator& op, void* const* xs, const void* b, int 
 }
 SolveResult dev_cg_mixed(const DevOperator& op, void* x, const void* b, const SolveOpts& o, const MixedOpts& m) {
   // resident where the system fits, unless a launch form was asked for
-  RsGeom g;
-  if (o.max_iter > 0 && m.sstep == 0 && sstep_default() == 2 && sstep_rows() == 0 && sstep_form() < 0 &&
-      rs_fits(op, g)) {
-    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_MIXED, m, g)) return *r;
-  }
+  if (m.sstep == 0 && sstep_default() == 2 && sstep_rows() == 0 && sstep_form() < 0)
+    if (auto r = rs_solve(op, x, b, o, RSF_MIXED, m)) return *r;
   if (!real_op(op) && (m.sstep ? m.sstep : sstep_default()) == 2 && sscg_fits(op)) {
     const int rows = sstep_rows_for(op.lx, op.ly);  // 0: the one-iteration form for this size
     if (rows > 0) return sscg_impl(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, m, rows);
@@ -2583,9 +2624,7 @@ SolveResult dev_cg_mixed(const DevOperator& op, void* x, const void* b, const So
 }
 SolveResult dev_cg_fused(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
   MixedOpts m;
-  RsGeom g;
-  if (o.max_iter > 0 && !o.per_launch && !real_op(op) && rs_fits(op, g))
-    if (auto r = rs_solve(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, RS_ONE, m, g)) return *r;
+  if (auto r = rs_solve(op, x, b, o, RSF_FUSED, m)) return *r;
   if (real_op(op))
     return fastcg_impl<double, double, false>(op, static_cast<double*>(x), static_cast<const double*>(b), o, m);
   return fastcg_impl<c128, c128, false>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, m);

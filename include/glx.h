@@ -443,10 +443,11 @@ int glx_dev_eo_reconstruct(glx_lattice lat, double mass, double* x_dev, const do
  * replayed (default 0: measured slightly slower than direct launches). */
 int glx_set_tuning(int group, int use_graph);
 /* Resident solves (no reference counterpart): where a system fits the chip's
- * registers, one launch keeps it there and runs every iteration (CG on D^dag D
- * and the even/odd solves, up to about 1020 x 1020 sites; the mixed solver up
- * to the next reliable update), with the numbers of a launch per iteration up
- * to the rounding of sums and hops.  on = 0: a launch per iteration always.
+ * registers, one launch keeps it there and runs the whole solve (CG on D^dag D
+ * and the even/odd solves, up to about 1020 x 1020 sites; CG on the Laplacians
+ * and BiCGStab on D, D^dag and the complex Laplacians, up to about 950 x 950
+ * and 850 x 850), with the numbers of a launch per iteration up to the
+ * rounding of sums and hops.  on = 0: a launch per iteration always.
  * spins: how often a block polls for another block's value before the launch
  * gives up and the solve is repeated with a launch per iteration (0: the
  * default, about a second).  A launch form chosen by glx_set_sstep or

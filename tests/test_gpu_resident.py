@@ -9,7 +9,7 @@ import threading
 import numpy as np
 import pytest
 
-from helpers import ENVELOPE, eo_envelope, lattice_inputs, relerr
+from helpers import ENVELOPE, bicgstab_envelope, eo_envelope, lattice_inputs, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -107,6 +107,48 @@ def test_even_odd(glx, orc, lx, ly, method):
     info, _ = glx.dev_solve_staggered_eo(lat, m, dx, db, method)
     assert info.success
     assert relerr(dx.download(), xs) <= ENVELOPE * err
+
+
+HOP_SIZES = [(2, 8), (7, 9), (62, 8), (63, 23), (64, 64), (130, 70), (97, 301), (300, 520)]
+
+
+@pytest.mark.parametrize("op", ["laplace_real", "laplace", "laplace_u1"])
+@pytest.mark.parametrize("lx,ly", HOP_SIZES)
+def test_one_hop_cg_matches_oracle(glx, orc, lx, ly, op):
+    """CG on the Laplacians through the host interface: the oracle's
+    iterations (one apart where the last residual is within rounding of the
+    tolerance), and |x - x*| <= |r| / m^2 with m^2 = 0.05 the gap."""
+    links, bc, br = lattice_inputs(orc, lx, ly, beta=6.25, seed=500 + lx + ly)
+    b = br if op == "laplace_real" else bc
+    kw = dict(links=links, mass=0.05, lx=lx, ly=ly, max_iter=5000)
+    xs, _ = orc.solve("cg", op, b, None, eps=1e-13, **kw)
+    xo, io = orc.solve("cg", op, b, None, eps=1e-10, **kw)
+    xg, ig = glx.minv_vector_cg(op, b, eps=1e-10, **kw)
+    assert ig.success and abs(ig.iter - io.iter) <= 1 and ig.ops_count == ig.iter + 2
+    if ig.iter == io.iter:
+        assert relerr(xg, xo) < 1e-11
+    r = b - orc.apply(op, xg, links, 0.05, lx, ly)
+    assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(b)
+    assert np.linalg.norm(xg - xs) <= 1.01e-10 * np.linalg.norm(b) / 0.05
+
+
+@pytest.mark.parametrize("op,mass", [("staggered", 0.2), ("staggered_dagger", 0.2), ("laplace_u1", 0.05), ("laplace", 0.05)])
+@pytest.mark.parametrize("lx,ly", HOP_SIZES)
+def test_one_hop_bicgstab(glx, orc, lx, ly, op, mass):
+    """BiCGStab's path depends on rounding: iterations within the range of the
+    oracle's on b and eight 1-ulp perturbations of it (97 x 301, laplace: 86 to
+    97), widened by its own width on either side; the true residual as
+    reported."""
+    links, b, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=600 + lx + ly)
+    kw = dict(links=links, mass=mass, lx=lx, ly=ly, max_iter=5000)
+    xg, ig = glx.minv_vector_bicgstab(op, b, eps=1e-10, **kw)
+    _, _, its, _ = bicgstab_envelope(orc, op, b, dict(kw, eps=1e-10))
+    width = max(2, its.max() - its.min())
+    assert ig.success and ig.ops_count == 2 * ig.iter + 2
+    assert its.min() - width <= ig.iter <= its.max() + width
+    r = b - orc.apply(op, xg, links, mass, lx, ly)
+    assert np.linalg.norm(r) <= 1e-9 * np.linalg.norm(b)
+    assert abs(np.sqrt(ig.resSq) - np.linalg.norm(r)) <= 1e-12 * np.linalg.norm(b)
 
 
 def test_guess_stop_and_zero(glx, orc):
