@@ -1,6 +1,7 @@
-// glx_reshop.hip -- the instances of the one-hop resident kernels (glx_reshop.h).
+// glx_reshop.hip -- the instances of the one-hop resident kernels
+// (glx_reshop.h) and of the multishift one (glx_rescgm.h).
 #include "glx_reshop.h"
-#include "glx_resident.h"
+#include "glx_rescgm.h"
 
 namespace glx {
 
@@ -46,6 +47,11 @@ void hop_bicgstab(hipStream_t st, const RsGeom& g, const RsSolve& so) {
 }
 }  // namespace
 
+void rs_launch_cg_m(hipStream_t st, const RsGeom& g, const RsSolve& so, const RsShiftSet& sh) {
+  rs_fill(st, so, rs_exchange_words(g, 2, 2));
+  hipLaunchKernelGGL(k_rs_cgm, dim3(g.nsx * g.nsy), dim3(kRsThreads), 0, st, g, so, sh);
+  GLX_CHECK_LAUNCH();
+}
 void rs_launch_hop_cg(hipStream_t st, const RsGeom& g, bool cplx, const RsSolve& so) {
   rs_fill(st, so, rs_exchange_words(g, cplx ? 2 : 1, 1));
   if (cplx) hop_cg<c128>(st, g, so);

@@ -56,19 +56,169 @@ struct RsShared {
   T h[kX ? 2 : 1][RS_NHALO][kX ? 64 : 1];
 };
 
+// D^dag D on a tile: its links, and the edge waves' halo values.
+template <class T, int R>
+struct RsNormal {
+  using Re = typename Real<T>::type;
+  using Sh = RsShared<T, R>;
+  using Tile = RsTile<T, R, 2>;
+  static constexpr int NW = kRsWaves;
+  Sh& sh;
+  const Tile& t;
+  Re m2;
+  T ux[R], uy[R], uxm[sizeof(T) == 8 ? R : 1];
+  T uyt_reg, hreg[Sh::kX ? 1 : RS_NHALO];
+
+  __device__ __forceinline__ T& hal(int v) {  // (edge waves only)
+    if constexpr (Sh::kX) return sh.h[t.top ? 0 : 1][v][t.lane];
+    else return hreg[v];
+  }
+  // U_y of the row above the run
+  __device__ __forceinline__ T& uyt() {
+    if constexpr (Sh::kR != 0) return sh.uyt[threadIdx.x];
+    else return uyt_reg;
+  }
+  __device__ __forceinline__ T uxm_of(int j) const { return uxm[sizeof(T) == 8 ? j : 0]; }
+
+  // loads the links: the run's, U_y above it and, on the edge waves, those of
+  // the nearest row beyond the tile with U_y of the row below it
+  __device__ __forceinline__ RsNormal(Sh& sh_, const Tile& t_, const RsLinks& lk, double mass)
+      : sh(sh_), t(t_), m2(Re(mass * mass)) {
+    const Re ey = (t.xg & 1) ? Re(-0.5) : Re(0.5);
+    const T b = zero_of<T>();
+    uxm[0] = b;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      ux[j] = uy[j] = b;
+      if (t.valid) rs_links<Re>(lk, (t.yw + j) * t.lx + t.xg, Re(0.5), ey, ux[j], uy[j]);
+      if constexpr (sizeof(T) == 8) uxm[j] = rs_shift<kDwPrev>(ux[j]);
+    }
+    T a, ux0 = b, uy0 = b, uy1 = b, uyw = b;
+    if (t.valid) {
+      rs_links<Re>(lk, t.wrapy(t.yw - 1) * t.lx + t.xg, Re(0.5), ey, a, uyw);
+      if (t.edge) {
+        rs_links<Re>(lk, t.yh[0] * t.lx + t.xg, Re(0.5), ey, ux0, uy0);
+        rs_links<Re>(lk, t.yh[1] * t.lx + t.xg, Re(0.5), ey, a, uy1);
+        if (!t.top) uy1 = uy[R - 1];
+      }
+    }
+    uyt_reg = b;
+    uyt() = uyw;
+    if (t.edge || !Sh::kX) {
+#pragma unroll
+      for (int v = 0; v < RS_UXH; v++) hal(v) = b;
+      hal(RS_UXH) = ux0;
+      hal(RS_UYH) = uy0;
+      hal(RS_UYHM) = uy1;
+    }
+  }
+
+  // ap = D^dag D p (p with its rim lanes, and the halo rows RS_PH of the edge
+  // waves): q = K p in ap, then m^2 p - K q in its place; f(j, ap_j) per row
+  template <class F>
+  __device__ __forceinline__ void apply(const T (&p)[R], T (&ap)[R], F f) {
+    const int lane = t.lane, wave = t.wave;
+    const bool top = t.top;
+    sh.v[0][wave][0][lane] = p[0];
+    sh.v[0][wave][1][lane] = p[R - 1];
+    __syncthreads();
+    T qh = zero_of<T>(), p0 = qh;
+    if (t.edge) {
+      p0 = hal(RS_PH);
+      const T p1 = hal(RS_PH + 1), uh = hal(RS_UXH);
+      qh = rs_hop(p0, top ? p1 : p[R - 1], top ? p[0] : p1, uh, rs_shift<kDwPrev>(uh), hal(RS_UYH), hal(RS_UYHM));
+    }
+    T up = top ? p0 : sh.v[0][top ? 0 : wave - 1][1][lane];
+    T below = wave == NW - 1 ? p0 : sh.v[0][wave + 1 < NW ? wave + 1 : wave][0][lane];
+    // (the scheduling fences keep the FP64 rows apart: interleaved, their
+    // temporaries spill the links)
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
+      ap[j] = rs_hop(p[j], j ? p[j ? j - 1 : 0] : up, j + 1 < R ? p[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j),
+                     uy[j], j ? uy[j ? j - 1 : 0] : uyt());
+    }
+    if constexpr (Sh::kV == 1) __syncthreads();
+    sh.v[Sh::kV - 1][wave][0][lane] = ap[0];
+    sh.v[Sh::kV - 1][wave][1][lane] = ap[R - 1];
+    __syncthreads();
+    up = top ? qh : sh.v[Sh::kV - 1][top ? 0 : wave - 1][1][lane];
+    below = wave == NW - 1 ? qh : sh.v[Sh::kV - 1][wave + 1 < NW ? wave + 1 : wave][0][lane];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
+      const T q = ap[j];
+      ap[j] = rs_mhop(m2, p[j], q, up, j + 1 < R ? ap[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j), uy[j],
+                      j ? uy[j ? j - 1 : 0] : uyt());
+      up = q;
+      f(j, ap[j]);
+    }
+  }
+};
+
+// out = b - (D^dag D + sigma) x in FP64 from memory (own lanes), with |out|^2
+// and |b|^2 of the counted rows in s2: a march down the wave's rows, at step i
+// the loads of row i - 2 of the run, q = K x on the row before it, A x on the
+// one before that.  at(y): the vectors' index of the lane's column in row y,
+// or -1 where a compact vector has none.
+template <class T, int R, class At>
+__device__ __forceinline__ void rs_normal_residual(const RsTile<T, R, 2>& t, const c128* u64, double mass, double sigma,
+                                                   const c128* x, const c128* b, At at, T (&out)[R],
+                                                   double (&s2)[2]) {
+  const double m2d = mass * mass + sigma;
+  const double ed = (t.xg & 1) ? -0.5 : 0.5;
+  const c128 z{0.0, 0.0};
+  c128 xa = z, xb = z, qa = z, qb = z, u1x = z, u1y = z, u2x = z, u2y = z, u3y = z;
+  s2[0] = s2[1] = 0.0;
+#pragma unroll 1
+  for (int i4 = 0; i4 < R + 4; i4++) {
+    const int y = t.wrapy(t.yw - 2 + i4), i = at(y);
+    c128 xc = z, ucx = z, ucy = z;
+    if (t.valid) {
+      if (i >= 0) xc = rs_read<c128>(reinterpret_cast<const unsigned long long*>(x + i));
+      rs_links<double>(RsLinks{u64, nullptr, 0}, y * t.lx + t.xg, 0.5, ed, ucx, ucy);
+    }
+    const c128 qc = rs_hop(xb, xa, xc, u1x, z, u1y, u2y);
+    if (i4 >= 4) {
+      const c128 ax = rs_mhop(m2d, xa, qb, qa, qc, u2x, z, u2y, u3y);
+      const int j = i4 - 4, ib = at(t.yw + j);
+      c128 d = z;
+      if (t.own && ib >= 0) {
+        const c128 bv = b[ib];
+        d = bv - ax;
+        if (t.counts(j)) {
+          s2[0] += norm2(d);
+          s2[1] += norm2(bv);
+        }
+      }
+      T dr;
+      cvt(dr, d);
+#pragma unroll
+      for (int jj = 0; jj < R; jj++)
+        if (jj == j) out[jj] = dr;
+    }
+    qa = qb;
+    qb = qc;
+    xa = xb;
+    xb = xc;
+    u3y = u2y;
+    u2x = u1x;
+    u2y = u1y;
+    u1x = ucx;
+    u1y = ucy;
+  }
+}
+
 template <class T, int R, int M>
 __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
   using Re = typename Real<T>::type;
   using A = typename std::conditional<M == RS_REF, T, Re>::type;  // alpha: complex in the reference's order
   using Sh = RsShared<T, R>;
-  constexpr int NW = kRsWaves;
   __shared__ Sh sh;
 
   RsTile<T, R, 2> t(sh.ex, g, so.ring, so.lines, so.spins);
-  const int lane = t.lane, wave = t.wave, lx = t.lx, yw = t.yw, xg = t.xg;
-  const bool top = t.top, edge = t.edge, valid = t.valid, own = t.own;
-  const Re ey = (xg & 1) ? Re(-0.5) : Re(0.5);
-  const Re m2 = Re(so.mass * so.mass);
+  const int lx = t.lx, yw = t.yw, xg = t.xg;
+  const bool edge = t.edge, own = t.own;
   // a vector's entry at (xg, y), or -1 where a compact vector has none
   // (the column passes through an empty asm statement, as in RsTile::slot)
   auto at = [&](int y) -> int {
@@ -77,7 +227,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     if (!so.eo) return y * lx + x;
     return ((x + y) & 1) ? -1 : y * (lx >> 1) + (x >> 1);
   };
-  T rv_[R - Sh::kR], p[R], ap[R], ux[R], uy[R], xr[Sh::kX ? 1 : R], uxm[sizeof(T) == 8 ? R : 1];
+  RsNormal<T, R> op(sh, t, so.lk, so.mass);
+  T rv_[R - Sh::kR], p[R], ap[R], xr[Sh::kX ? 1 : R];
   auto xref = [&](int j) -> T& {
     if constexpr (Sh::kX) return sh.x[j][threadIdx.x];
     else return xr[j];
@@ -88,52 +239,16 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     }
     return rv_[j < R - Sh::kR ? j : 0];
   };
-  auto uxm_of = [&](int j) -> T { return uxm[sizeof(T) == 8 ? j : 0]; };
-  uxm[0] = zero_of<T>();
+  auto hal = [&](int v) -> T& { return op.hal(v); };
 #pragma unroll
   for (int j = 0; j < R; j++) {
-    rref(j) = p[j] = ap[j] = ux[j] = uy[j] = zero_of<T>();
+    rref(j) = p[j] = ap[j] = zero_of<T>();
     T x = zero_of<T>();
-    if (valid) {
-      rs_links<Re>(so.lk, (yw + j) * lx + xg, Re(0.5), ey, ux[j], uy[j]);
-      if constexpr (M != RS_MIXED) {
-        const int i = at(yw + j);
-        if (own && i >= 0) x = so.x[i];
-      }
+    if constexpr (M != RS_MIXED) {
+      const int i = at(yw + j);
+      if (own && i >= 0) x = so.x[i];
     }
     xref(j) = x;
-    if constexpr (sizeof(T) == 8) uxm[j] = rs_shift<kDwPrev>(ux[j]);
-  }
-  // U_y of the row above the run; on the edge waves the two rows beyond the
-  // tile, nearest first (y0 - 1, y0 - 2 or y0 + L, y0 + L + 1), and the
-  // nearest one's links with U_y of the row below it
-  T uyt_reg = zero_of<T>(), hreg[Sh::kX ? 1 : RS_NHALO];
-  auto hal = [&](int v) -> T& {  // (edge waves only)
-    if constexpr (Sh::kX) return sh.h[top ? 0 : 1][v][lane];
-    else return hreg[v];
-  };
-  auto uyt = [&]() -> T& {
-    if constexpr (Sh::kR != 0) return sh.uyt[threadIdx.x];
-    else return uyt_reg;
-  };
-  {
-    T a, b = zero_of<T>(), ux0 = b, uy0 = b, uy1 = b, uyw = b;
-    if (valid) {
-      rs_links<Re>(so.lk, t.wrapy(yw - 1) * lx + xg, Re(0.5), ey, a, uyw);
-      if (edge) {
-        rs_links<Re>(so.lk, t.yh[0] * lx + xg, Re(0.5), ey, ux0, uy0);
-        rs_links<Re>(so.lk, t.yh[1] * lx + xg, Re(0.5), ey, a, uy1);
-        if (!top) uy1 = uy[R - 1];
-      }
-    }
-    uyt() = uyw;
-    if (edge || !Sh::kX) {
-#pragma unroll
-      for (int v = 0; v < RS_UXH; v++) hal(v) = b;
-      hal(RS_UXH) = ux0;
-      hal(RS_UYH) = uy0;
-      hal(RS_UYHM) = uy1;
-    }
   }
   if (threadIdx.x == 0) sh.ex.bad = 0;
 
@@ -154,51 +269,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
   __syncthreads();
   for (;;) {
     {
-      // ---- r = b - A x with FP64 links, a march down the wave's rows: at
-      // step i4 the loads of row i4 - 2 of the run, q = K x on the row before
-      // it, A x on the one before that
-      const double m2d = so.mass * so.mass;
-      const double ed = (xg & 1) ? -0.5 : 0.5;
-      const c128 z{0.0, 0.0};
-      c128 xa = z, xb = z, qa = z, qb = z, u1x = z, u1y = z, u2x = z, u2y = z, u3y = z;
-      double s2[2] = {0.0, 0.0};
-#pragma unroll 1
-      for (int i4 = 0; i4 < R + 4; i4++) {
-        const int y = t.wrapy(yw - 2 + i4), i = at(y);
-        c128 xc = z, ucx = z, ucy = z;
-        if (valid) {
-          if (i >= 0) xc = rs_read<c128>(reinterpret_cast<const unsigned long long*>(so.x + i));
-          rs_links<double>(RsLinks{so.u64, nullptr, 0}, y * lx + xg, 0.5, ed, ucx, ucy);
-        }
-        const c128 qc = rs_hop(xb, xa, xc, u1x, z, u1y, u2y);
-        if (i4 >= 4) {
-          const c128 ax = rs_mhop(m2d, xa, qb, qa, qc, u2x, z, u2y, u3y);
-          const int j = i4 - 4, ib = at(yw + j);
-          c128 d = z;
-          if (own && ib >= 0) {
-            const c128 bv = so.b[ib];
-            d = bv - ax;
-            if (t.counts(j)) {
-              s2[0] += norm2(d);
-              s2[1] += norm2(bv);
-            }
-          }
-          T dr;
-          cvt(dr, d);
-#pragma unroll
-          for (int jj = 0; jj < R; jj++)
-            if (jj == j) ap[jj] = dr;
-        }
-        qa = qb;
-        qb = qc;
-        xa = xb;
-        xb = xc;
-        u3y = u2y;
-        u2x = u1x;
-        u2y = u1y;
-        u1x = ucx;
-        u1y = ucy;
-      }
+      double s2[2];
+      rs_normal_residual<T, R>(t, so.u64, so.mass, 0.0, so.x, so.b, at, ap, s2);
       t.publish(ap, e, s2, c);
       if (!t.collect(ap, [&](int h, T v) { hal(RS_RH + h) = v; }, e, s2, c)) return give_up();
       e++;
@@ -244,45 +316,11 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
         hal(RS_PH + h) = rs_axpy(be, hal(RS_PH + h), rh);
       }
     }
-    sh.v[0][wave][0][lane] = p[0];
-    sh.v[0][wave][1][lane] = p[R - 1];
-
-    // ---- q = K p (in ap), then Ap = m^2 p - K q in its place
-    __syncthreads();
-    T qh = zero_of<T>(), p0 = qh;
-    if (edge) {
-      p0 = hal(RS_PH);
-      const T p1 = hal(RS_PH + 1), uh = hal(RS_UXH);
-      qh = rs_hop(p0, top ? p1 : p[R - 1], top ? p[0] : p1, uh, rs_shift<kDwPrev>(uh), hal(RS_UYH), hal(RS_UYHM));
-    }
-    T up = top ? p0 : sh.v[0][top ? 0 : wave - 1][1][lane];
-    T below = wave == NW - 1 ? p0 : sh.v[0][wave + 1 < NW ? wave + 1 : wave][0][lane];
-    // (the scheduling fences keep the FP64 rows apart: interleaved, their
-    // temporaries spill the links)
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-      if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
-      ap[j] = rs_hop(p[j], j ? p[j ? j - 1 : 0] : up, j + 1 < R ? p[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j),
-                     uy[j], j ? uy[j ? j - 1 : 0] : uyt());
-    }
-    if constexpr (Sh::kV == 1) __syncthreads();
-    sh.v[Sh::kV - 1][wave][0][lane] = ap[0];
-    sh.v[Sh::kV - 1][wave][1][lane] = ap[R - 1];
-    __syncthreads();
-    up = top ? qh : sh.v[Sh::kV - 1][top ? 0 : wave - 1][1][lane];
-    below = wave == NW - 1 ? qh : sh.v[Sh::kV - 1][wave + 1 < NW ? wave + 1 : wave][0][lane];
     constexpr int N1 = M == RS_REF ? 2 : 4;
     double v1[N1];
 #pragma unroll
     for (int i = 0; i < N1; i++) v1[i] = 0.0;
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-      if constexpr (Sh::kX) __builtin_amdgcn_sched_barrier(0);
-      const T q = ap[j];
-      const T v = rs_mhop(m2, p[j], q, up, j + 1 < R ? ap[j + 1 < R ? j + 1 : j] : below, ux[j], uxm_of(j), uy[j],
-                          j ? uy[j ? j - 1 : 0] : uyt());
-      up = q;
-      ap[j] = v;
+    op.apply(p, ap, [&](int j, T v) {
       if (t.counts(j)) {
         const double pr = p[j].re, pi = p[j].im, ar = v.re, ai = v.im;
         v1[0] = __builtin_fma(pr, ar, __builtin_fma(pi, ai, v1[0]));
@@ -296,7 +334,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
           v1[3] = __builtin_fma(rr, rr, __builtin_fma(ri, ri, v1[3]));
         }
       }
-    }
+    });
 #pragma unroll
     for (int i = 0; i < N1; i++) v1[i] = own ? v1[i] : 0.0;
     t.publish(ap, e, v1, c);
@@ -409,6 +447,17 @@ void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so);
 constexpr int kRsMostRowsHop = 8, kRsMostRowsBicg = 6;
 void rs_launch_hop_cg(hipStream_t st, const RsGeom& g, bool cplx, const RsSolve& so);
 void rs_launch_hop_bicgstab(hipStream_t st, const RsGeom& g, int sb, const RsSolve& so);
+
+// Multishift CG (glx_rescgm.h), its kernel one row per wave.
+constexpr int kRsShifts = 16;  // shifts a resident solve may have
+struct RsShiftSet {
+  int n, freq;  // shifts, iterations between convergence checks
+  double shift[kRsShifts];
+  c128* x[kRsShifts];
+  double* res;  // [n] |(A + shift) x - b|^2
+};
+bool rs_plan_one_row(int lx, int ly, int halo, RsGeom& g);
+void rs_launch_cg_m(hipStream_t st, const RsGeom& g, const RsSolve& so, const RsShiftSet& sh);
 
 // The resident blocks of every solve in flight on a device, over all host
 // threads, stay within its CUs, one block each: a solve waits here until its

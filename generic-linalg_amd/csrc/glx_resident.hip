@@ -115,6 +115,14 @@ bool rs_plan(int lx, int ly, int halo, int most_rows, RsGeom& g) {
   return false;
 }
 
+bool rs_plan_one_row(int lx, int ly, int halo, RsGeom& g) {
+  if (lx < 2 * halo || ly < kRsWaves || long(lx) * ly > (1L << 24)) return false;
+  const int nsx = (lx + rs_cols(halo) - 1) / rs_cols(halo), nsy = (ly + kRsWaves - 1) / kRsWaves;
+  if (long(nsx) * nsy > std::min(kRsMaxBlocks, device_cus(current_device()))) return false;
+  g = RsGeom{lx, ly, nsx, nsy, 1};
+  return true;
+}
+
 void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so) {
   if (mode == RS_REF) launch<c128, RS_REF>(st, g, so);
   else if (mode == RS_ONE) launch<c128, RS_ONE>(st, g, so);

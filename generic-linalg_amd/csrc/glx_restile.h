@@ -273,10 +273,11 @@ __device__ __forceinline__ double rs_block_words(const double (*w)[4]) {
   return rs_xor16(rs_quads(w[(lane >> 2) & 7][lane & 3]));
 }
 
-// Adds ND values over the block and stores them to the block's line of
+// Adds ND values over block blk and stores them to the block's line of
 // reduction c, then empties its line of reduction c + 2.
 template <int ND>
-__device__ __forceinline__ void rs_publish(const double (&v)[ND], double (*sm)[4], unsigned long long* lines, int c) {
+__device__ __forceinline__ void rs_publish(const double (&v)[ND], double (*sm)[4], unsigned long long* lines, int c,
+                                           int blk) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const double t = rs_wave_words<ND>(v);
   if (lane < ND) sm[wave][lane] = t;
@@ -284,10 +285,10 @@ __device__ __forceinline__ void rs_publish(const double (&v)[ND], double (*sm)[4
   if (wave == 0) {
     const double b = rs_block_words(sm);
     if (lane < ND)
-      rs_store(lines + ((c & 3) * kRsMaxBlocks + blockIdx.x) * kRsLine + lane,
+      rs_store(lines + ((c & 3) * kRsMaxBlocks + blk) * kRsLine + lane,
                (unsigned long long)__double_as_longlong(b));
     // (all words: reduction c + 2 may have more of them than this one)
-    if (lane < 4) rs_store(lines + (((c + 2) & 3) * kRsMaxBlocks + blockIdx.x) * kRsLine + lane, kRsEmpty);
+    if (lane < 4) rs_store(lines + (((c + 2) & 3) * kRsMaxBlocks + blk) * kRsLine + lane, kRsEmpty);
   }
 }
 
@@ -312,7 +313,7 @@ struct RsTile {
   static constexpr int NW = kRsWaves, L = NW * R;
   using Sh = RsExShared<T, R, H>;
   Sh& sh;
-  int lane, wave, nblk, lx, ly;
+  int lane, wave, blk, nblk, lx, ly;  // blk of nblk: the system's blocks
   int x0, cols, y0, shared;  // shared: the first rows, which the band before stores and counts
   int yw;                    // the wave's first row
   int xg;                    // the lane's column (0 where not valid)
@@ -327,14 +328,14 @@ struct RsTile {
   int spins;
 
   __device__ __forceinline__ RsTile(Sh& sh_, const RsGeom& g, unsigned long long* ring_, unsigned long long* lines_,
-                                    int spins_)
-      : sh(sh_), ring(reinterpret_cast<char*>(ring_)), lines(lines_), spins(spins_) {
+                                    int spins_, int blk_ = blockIdx.x)
+      : sh(sh_), blk(blk_), ring(reinterpret_cast<char*>(ring_)), lines(lines_), spins(spins_) {
     lane = threadIdx.x & 63;
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    nblk = gridDim.x;
+    nblk = g.nsx * g.nsy;
     lx = g.lx;
     ly = g.ly;
-    const int sx = blockIdx.x % g.nsx, sy = blockIdx.x / g.nsx;
+    const int sx = blk % g.nsx, sy = blk / g.nsx;
     x0 = int(long(lx) * sx / g.nsx);
     cols = int(long(lx) * (sx + 1) / g.nsx) - x0;
     // every tile has L rows: the last band begins early and shares rows with
@@ -370,9 +371,9 @@ struct RsTile {
     mrow = lane / (2 * H);
     mcol = lane & (2 * H - 1);
     mover = lane < 2 * H * R;
-    const int row0 = blockIdx.x - sx;  // the band's first block
+    const int row0 = blk - sx;  // the band's first block
     const int left = row0 + (sx == 0 ? g.nsx - 1 : sx - 1), right = row0 + (sx == g.nsx - 1 ? 0 : sx + 1);
-    put_off = col_off(blockIdx.x, mcol);
+    put_off = col_off(blk, mcol);
     get_off = col_off(mcol < H ? left : right, mcol ^ H);
     scol = lane < 2 * H ? lane - H : lane - cols + H;  // a side lane's column of the 2 H
     rcol = lane < H ? lane : lane - cols;              // a rim lane's
@@ -419,7 +420,7 @@ struct RsTile {
     rs_stores_done();  // (the slots emptied since the last reduction)
     if (mover) rs_put<T>(col_word(e, put_off), sh.rim[wave][mrow][mcol]);
     for_rows(e, [&](unsigned long long* q, int j) { rs_put<T>(q, v[j]); });
-    rs_publish(sums, sh.part, lines, c);
+    rs_publish(sums, sh.part, lines, c, blk);
     if (mover) rs_empty<T>(col_word(e + 2, put_off));
     for_rows(e + 2, [&](unsigned long long* q, int) { rs_empty<T>(q); });
   }
@@ -427,7 +428,7 @@ struct RsTile {
   template <int ND>
   __device__ __forceinline__ void publish(const double (&sums)[ND], int c) {
     rs_stores_done();  // (slots and lines emptied since the last reduction)
-    rs_publish(sums, sh.part, lines, c);
+    rs_publish(sums, sh.part, lines, c, blk);
   }
   // Collects ring use e into the rim lanes of v and, by halo(h, value) on the
   // edge waves, the halo rows (RING), and the totals of reduction c over all

@@ -2583,6 +2583,62 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, void* x, const 
   return res;
 }
 
+// Multishift CG on D^dag D: every shift's vectors in registers too.
+static std::optional<SolveResult> rs_solve_cg_m(const DevOperator& o, void* const* xs, const void* b, int n_shift,
+                                                const double* shifts, int resid_freq, bool worst_first,
+                                                const SolveOpts& opt) {
+  RsGeom g;
+  if (!resident_on() || o.kind != OP_STAG_NORMAL || !o.tiled() || !o.u64 || opt.max_iter <= 0 || worst_first ||
+      n_shift < 1 || n_shift > kRsShifts || resid_freq < 1 || !rs_plan_one_row(o.lx, o.ly, 2, g))
+    return std::nullopt;
+  hipStream_t st = opt.stream;
+  RsSolve so{};
+  so.b = static_cast<const c128*>(b);
+  so.u64 = o.u64;
+  so.lk = RsLinks{o.u64, nullptr, LINKS_F64};
+  so.mass = o.mass;
+  so.eps = opt.eps;
+  so.max_iter = opt.max_iter;
+  so.spins = resident_spins();
+  DevBuf ex(size_t(rs_exchange_words(g, rs_words<c128>(), 2)) * 8), out(sizeof(RsOut)), res(sizeof(double) * n_shift);
+  DevBuf hist(opt.want_hist ? size_t(opt.max_iter) * sizeof(double) : 0);
+  so.lines = ex.as<unsigned long long>();
+  so.ring = so.lines + long(kRsBufs) * kRsMaxBlocks * kRsLine;
+  so.out = out.as<RsOut>();
+  so.hist = hist.as<double>();
+  RsShiftSet sh{};
+  sh.n = n_shift;
+  sh.freq = resid_freq;
+  sh.res = res.as<double>();
+  for (int k = 0; k < n_shift; k++) {
+    sh.shift[k] = shifts[k];
+    sh.x[k] = static_cast<c128*>(xs[k]);
+  }
+  RsOut h{};
+  SolveResult r;
+  r.resSqmrhs.resize(n_shift);
+  {
+    RsReserve slots(g.nsx * g.nsy);
+    rs_launch_cg_m(st, g, so, sh);
+    GLX_HIP(hipMemcpyAsync(&h, so.out, sizeof(h), hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipMemcpyAsync(r.resSqmrhs.data(), res.get(), sizeof(double) * n_shift, hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipStreamSynchronize(st));
+  }
+  if (h.err || !h.done) return std::nullopt;
+  r.name = "CG-M";
+  r.success = h.kfinal != opt.max_iter - 1;
+  r.iter = h.kfinal + 1;
+  r.ops_count = 1 + h.kfinal + n_shift;
+  r.resSq = 0.0;
+  r.bsqrt = h.bsqrt;
+  if (opt.want_hist) {
+    r.relres_hist.resize(r.iter);
+    GLX_HIP(hipMemcpyAsync(r.relres_hist.data(), so.hist, sizeof(double) * r.iter, hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipStreamSynchronize(st));
+  }
+  return r;
+}
+
 // ============================================================ dispatch ====
 static bool real_op(const DevOperator& o) {
   return o.is_host() ? !o.host_complex : o.kind == OP_LAPLACE_REAL;
@@ -2604,6 +2660,7 @@ SolveResult dev_gcr(const DevOperator& op, void* x, const void* b, const SolveOp
 }
 SolveResult dev_cg_m(const DevOperator& op, void* const* xs, const void* b, int n_shift, const double* shifts,
                      int resid_freq_check, bool worst_first, const SolveOpts& o) {
+  if (auto r = rs_solve_cg_m(op, xs, b, n_shift, shifts, resid_freq_check, worst_first, o)) return *r;
   if (real_op(op))
     return cg_m_impl<double>(op, reinterpret_cast<double* const*>(xs), static_cast<const double*>(b), n_shift, shifts,
                              resid_freq_check, worst_first, o);

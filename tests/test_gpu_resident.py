@@ -151,6 +151,43 @@ def test_one_hop_bicgstab(glx, orc, lx, ly, op, mass):
     assert abs(np.sqrt(ig.resSq) - np.linalg.norm(r)) <= 1e-12 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("lx,ly,n_shift,freq", [(4, 8, 1, 1), (4, 8, 16, 10), (60, 9, 5, 3), (61, 23, 16, 10),
+                                                (130, 70, 2, 7), (200, 144, 12, 10)])
+def test_multishift_matches_oracle(glx, orc, lx, ly, n_shift, freq):
+    """Every shift's solution and residual, and the iterations (a check apart
+    where a shift crosses the tolerance within rounding)."""
+    m = 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    shifts = 10.0 ** np.linspace(-3.0, 2.5, n_shift)
+    kw = dict(links=links, mass=m, lx=lx, ly=ly, resid_freq_check=freq, max_iter=5000, eps=1e-10)
+    X, io, _, _ = orc.cg_m("staggered_normal", b, shifts, **kw)
+    xs = [glx.DeviceArray(b) for _ in shifts]  # (what they hold is overwritten)
+    ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, resid_freq_check=freq, max_iter=5000)
+    assert ig.success and abs(ig.iter - io.iter) <= freq and ig.ops_count == ig.iter + n_shift
+    nb = np.linalg.norm(b)
+    for k, s in enumerate(shifts):
+        x = xs[k].download()
+        r = b - orc.apply("staggered_normal", x, links, m, lx, ly) - s * x
+        assert abs(np.sqrt(ig.resSqmrhs[k]) - np.linalg.norm(r)) <= 1e-12 * nb
+        assert np.linalg.norm(r) <= 2e-10 * nb
+        # both are within |r| / (m^2 + s) of the solution
+        assert np.linalg.norm(x - X[k]) <= 4e-10 * nb / (m * m + s)
+
+
+def test_multishift_stops_at_max_iter(glx, orc):
+    lx, ly, m = 61, 23, 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+    shifts = [0.0, 0.01, 1.0]
+    for stop in (1, 2, 11):
+        X, io, _, _ = orc.cg_m("staggered_normal", b, shifts, links=links, mass=m, lx=lx, ly=ly, resid_freq_check=10,
+                               max_iter=stop, eps=1e-10)
+        xs = [glx.DeviceArray(np.zeros_like(b)) for _ in shifts]
+        ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, max_iter=stop)
+        assert (ig.iter, ig.success, ig.ops_count) == (io.iter, io.success, io.ops_count)
+        for x, xo in zip(xs, X):
+            assert relerr(x.download(), xo) < 1e-12
+
+
 def test_guess_stop_and_zero(glx, orc):
     """A guess that is nearly the solution, max_iter stops, b = 0."""
     lx, ly, m = 130, 70, 0.1
