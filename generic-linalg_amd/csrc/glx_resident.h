@@ -424,6 +424,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
 // run resident, and the polls a wait may take before it gives up.
 void set_resident(int on, int spins);
 bool resident_on();
+int rs_cus();  // CUs of the current device
 int resident_spins();
 
 // The tiling a system would run resident with on the current device, for an

@@ -87,6 +87,7 @@ void set_resident(int on, int spins) {
   g_on.store(on ? 1 : 0);
   g_spins.store(spins > 0 ? spins : kSpins);
 }
+int rs_cus() { return device_cus(current_device()); }
 bool resident_on() { return g_on.load() != 0; }
 int resident_spins() { return g_spins.load(); }
 

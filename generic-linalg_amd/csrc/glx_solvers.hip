@@ -13,6 +13,7 @@
 // zeta, ...) are computed on the device by the reduction finalisers and read
 // by the next kernel; the host reads the 16-byte control word once per chunk.
 #include "glx_solvers.h"
+#include "glx_resgcr.h"
 #include "glx_resident.h"
 #include "glx_sstep.h"
 #include "glx_sswave.h"
@@ -248,9 +249,9 @@ struct Work {
 // kernels of iteration k; `pause(m)` handles a device-requested pause
 // (done == 2) and returns the next iteration index.
 template <class Enq, class Pause>
-Mirror run_loop(Work& w, int max_iter, int chunk, Enq enq, Pause pause) {
+Mirror run_loop(Work& w, int max_iter, int chunk, Enq enq, Pause pause, int first = 0) {
   PinnedSlots& pin = pinned();
-  int next = 0;
+  int next = first;
   int cur = 0;
   bool inflight = false;
   Mirror m{0, 0, -1, 0};
@@ -945,8 +946,17 @@ struct PtGcrComb {
   }
 };
 
+// A solve that iterations elsewhere have brought to k (k = 0: none): r and x
+// after iteration k - 1, which did not converge, and the directions so far.
+struct GcrStart {
+  int k = 0;
+  double bsqrt = 0.0;
+  DevBuf r, norms, hist;
+  std::vector<DevBuf> store;      // per kRgDirs directions [p_j, A p_j]
+};
+
 template <class T>
-SolveResult gcr_impl(const DevOperator& o, T* x, const T* b, const SolveOpts& opt) {
+SolveResult gcr_impl(const DevOperator& o, T* x, const T* b, const SolveOpts& opt, const GcrStart& from) {
   const int n = o.size();
   Work w(opt.stream, stencil_blocks(std::max(o.lx, 1), std::max(o.ly, 1)), opt.max_iter, opt.want_hist);
   SolveState h;
@@ -954,6 +964,8 @@ SolveResult gcr_impl(const DevOperator& o, T* x, const T* b, const SolveOpts& op
   h.max_iter = opt.max_iter;
   h.eps = opt.eps;
   h.hist = w.hist.as<double>();
+  h.k = from.k;
+  h.bsqrt = from.bsqrt;
   w.upload(h);
   const size_t vb = n * sizeof(T);
   const int cap = std::max(opt.max_iter, 0) + 1;
@@ -977,16 +989,10 @@ SolveResult gcr_impl(const DevOperator& o, T* x, const T* b, const SolveOpts& op
   };
   hp.reserve(cap);
   hap.reserve(cap);
-  add_dir();
-  apply_typed<T>(w.st, o, LINKS_F64, tmpB.as<T>(), x, w.ws(), kNoGate);
-  launch_point(w.st, n, PtGcrInit<T>{r, hp[0], b, tmpB.as<T>()}, FinBsqrt{w.ds}, w.ws(), kNoGate);
-  apply_typed<T>(w.st, o, LINKS_F64, hap[0], hp[0], w.ws(), kNoGate);
   c128* betas = betasB.as<c128>();
   double* norms = normsB.as<double>();
-  auto enq = [&](int k) {
-    launch_point(w.st, n, PtGcrAlpha<T>{hap[k], r}, FinGcrAlpha<T>{w.ds, norms, k}, w.ws(), w.done());
-    launch_point(w.st, n, PtGcrXR<T>{x, r, hp[k], hap[k], w.ds}, FinGcrNorm{w.ds}, w.ws(), w.done());
-    if (k == opt.max_iter - 1) return;  // the device stops here at the latest
+  // direction k + 1 from r
+  auto extend = [&](int k) {
     apply_typed<T>(w.st, o, LINKS_F64, ar, r, w.ws(), w.done());
     for (int j0 = 0; j0 <= k; j0 += kGcrGroup) {
       const int cnt = std::min(kGcrGroup, k + 1 - j0);
@@ -996,7 +1002,33 @@ SolveResult gcr_impl(const DevOperator& o, T* x, const T* b, const SolveOpts& op
     add_dir();
     launch_point(w.st, n, PtGcrComb<T>{ptab, aptab, betas, r, ar, k}, FinNone{}, w.ws(), w.done());
   };
-  Mirror m = run_loop(w, opt.max_iter, opt.chunk, enq, [](const Mirror&) { return -1; });
+  if (from.k == 0) {
+    add_dir();
+    apply_typed<T>(w.st, o, LINKS_F64, tmpB.as<T>(), x, w.ws(), kNoGate);
+    launch_point(w.st, n, PtGcrInit<T>{r, hp[0], b, tmpB.as<T>()}, FinBsqrt{w.ds}, w.ws(), kNoGate);
+    apply_typed<T>(w.st, o, LINKS_F64, hap[0], hp[0], w.ws(), kNoGate);
+  } else {
+    for (int j = 0; j < from.k; j++) {
+      hp.push_back(from.store[j / kRgDirs].as<T>() + size_t(2 * (j % kRgDirs)) * n);
+      hap.push_back(hp.back() + n);
+    }
+    auto copy = [&](void* to, const void* src, size_t bytes, hipMemcpyKind kind) {
+      GLX_HIP(hipMemcpyAsync(to, src, bytes, kind, w.st));
+    };
+    copy(ptab, hp.data(), sizeof(T*) * from.k, hipMemcpyHostToDevice);
+    copy(aptab, hap.data(), sizeof(T*) * from.k, hipMemcpyHostToDevice);
+    copy(r, from.r.get(), vb, hipMemcpyDeviceToDevice);
+    copy(norms, from.norms.get(), sizeof(double) * from.k, hipMemcpyDeviceToDevice);
+    if (opt.want_hist) copy(h.hist, from.hist.get(), sizeof(double) * from.k, hipMemcpyDeviceToDevice);
+    extend(from.k - 1);
+  }
+  auto enq = [&](int k) {
+    launch_point(w.st, n, PtGcrAlpha<T>{hap[k], r}, FinGcrAlpha<T>{w.ds, norms, k}, w.ws(), w.done());
+    launch_point(w.st, n, PtGcrXR<T>{x, r, hp[k], hap[k], w.ds}, FinGcrNorm{w.ds}, w.ws(), w.done());
+    if (k == opt.max_iter - 1) return;  // the device stops here at the latest
+    extend(k);
+  };
+  Mirror m = run_loop(w, opt.max_iter, opt.chunk, enq, [](const Mirror&) { return -1; }, from.k);
   SolveResult res;
   res.name = "GCR";
   const int kf = opt.max_iter > 0 ? m.kfinal : 0;
@@ -2639,6 +2671,80 @@ static std::optional<SolveResult> rs_solve_cg_m(const DevOperator& o, void* cons
   return r;
 }
 
+// GCR on the general stencil, a launch per kRgDirs iterations.  A solve that
+// needs more than kRgChunks launches leaves its state in `from`, to be
+// continued there with a launch per phase.
+static std::optional<SolveResult> rs_solve_gcr(const DevOperator& o, void* x, const void* b, const SolveOpts& opt,
+                                               GcrStart& from) {
+  RsGcr g{};
+  int m = 0;
+  if (o.is_host() || o.kind != OP_CST || opt.max_iter <= 0 || opt.per_launch || noalloc_scope() ||
+      !rg_plan(cst_dev(o, CS_ALL), g, m))
+    return std::nullopt;
+  hipStream_t st = opt.stream;
+  const int n = o.size();
+  const size_t vb = sizeof(c128) * n;
+  GcrStart s;
+  DevBuf xs(vb), out(sizeof(RsOut));
+  s.r = DevBuf(vb);
+  s.norms = DevBuf(sizeof(double) * kRgDirs * kRgChunks);
+  s.hist = DevBuf(opt.want_hist ? sizeof(double) * opt.max_iter : 0);
+  g.max_iter = opt.max_iter;
+  g.spins = resident_spins();
+  g.eps = opt.eps;
+  g.x = static_cast<c128*>(x);
+  g.b = static_cast<const c128*>(b);
+  g.xs = xs.as<c128>();
+  g.rs = s.r.as<c128>();
+  g.norms = s.norms.as<double>();
+  g.hist = s.hist.as<double>();
+  g.out = out.as<RsOut>();
+  RsOut h{};
+  for (int c = 0; c < kRgChunks && !h.done; c++) {
+    g.k0 = c * kRgDirs;
+    DevBuf ex;
+    try {
+      s.store.emplace_back(2 * vb * std::min(kRgDirs, opt.max_iter - g.k0));
+      ex = DevBuf(size_t(rg_exchange_words(g)) * 8);
+    } catch (const std::exception&) {
+      return std::nullopt;  // no room for this many directions at once
+    }
+    g.dir[c] = s.store.back().as<c128>();
+    g.lines = ex.as<unsigned long long>();
+    g.ring = g.lines + long(kRsBufs) * kRsMaxBlocks * kRsLine;
+    g.d1 = g.ring + long(kRsBufs) * 2 * n;
+    g.d2 = g.d1 + long(kRsBufs) * g.nblk * rg_words(g.k0);
+    {
+      RsReserve slots(g.nblk);
+      rg_launch(st, m, g);
+      GLX_HIP(hipMemcpyAsync(&h, g.out, sizeof(h), hipMemcpyDeviceToHost, st));
+      GLX_HIP(hipStreamSynchronize(st));
+    }
+    if (h.err) return std::nullopt;
+    if (c == 0) g.bsqrt = h.bsqrt;
+  }
+  if (!h.done) {
+    GLX_HIP(hipMemcpyAsync(x, g.xs, vb, hipMemcpyDeviceToDevice, st));
+    s.k = kRgDirs * kRgChunks;
+    s.bsqrt = g.bsqrt;
+    from = std::move(s);
+    return std::nullopt;
+  }
+  SolveResult res;
+  res.name = "GCR";
+  res.iter = h.kfinal + 1;
+  res.success = h.kfinal != opt.max_iter - 1;
+  res.ops_count = res.iter + 2;
+  res.resSq = h.resSq;
+  res.bsqrt = g.bsqrt;
+  if (opt.want_hist) {
+    res.relres_hist.resize(res.iter);
+    GLX_HIP(hipMemcpyAsync(res.relres_hist.data(), g.hist, sizeof(double) * res.iter, hipMemcpyDeviceToHost, st));
+    GLX_HIP(hipStreamSynchronize(st));
+  }
+  return res;
+}
+
 // ============================================================ dispatch ====
 static bool real_op(const DevOperator& o) {
   return o.is_host() ? !o.host_complex : o.kind == OP_LAPLACE_REAL;
@@ -2655,8 +2761,10 @@ SolveResult dev_bicgstab(const DevOperator& op, void* x, const void* b, const So
   return bicgstab_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o);
 }
 SolveResult dev_gcr(const DevOperator& op, void* x, const void* b, const SolveOpts& o) {
-  if (real_op(op)) return gcr_impl<double>(op, static_cast<double*>(x), static_cast<const double*>(b), o);
-  return gcr_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o);
+  GcrStart from;
+  if (auto r = rs_solve_gcr(op, x, b, o, from)) return *r;
+  if (real_op(op)) return gcr_impl<double>(op, static_cast<double*>(x), static_cast<const double*>(b), o, from);
+  return gcr_impl<c128>(op, static_cast<c128*>(x), static_cast<const c128*>(b), o, from);
 }
 SolveResult dev_cg_m(const DevOperator& op, void* const* xs, const void* b, int n_shift, const double* shifts,
                      int resid_freq_check, bool worst_first, const SolveOpts& o) {

@@ -447,7 +447,8 @@ int glx_set_tuning(int group, int use_graph);
  * and the even/odd solves, up to about 1020 x 1020 sites; CG on the Laplacians
  * and BiCGStab on D, D^dag and the complex Laplacians, up to about 950 x 950
  * and 850 x 850; multishift CG on D^dag D with up to 16 shifts and without
- * worst_first, up to about 340 x 340), with the numbers of a launch per iteration up to the
+ * worst_first, up to about 340 x 340; GCR on the general stencil up to about
+ * 65000 entries), with the numbers of a launch per iteration up to the
  * rounding of sums and hops.  on = 0: a launch per iteration always.
  * spins: how often a block polls for another block's value before the launch
  * gives up and the solve is repeated with a launch per iteration (0: the

@@ -188,6 +188,94 @@ def test_multishift_stops_at_max_iter(glx, orc):
             assert relerr(x.download(), xo) < 1e-12
 
 
+# lx, ly, nc, two: one site and one block; wraps onto itself; last blocks with
+# few sites; a site of 12 colours in 64 entries; two and four entries per lane;
+# more colours than lanes
+STENCILS = [(1, 1, 1, False), (6, 5, 1, False), (3, 2, 12, True), (16, 12, 4, True), (33, 31, 3, True),
+            (32, 32, 8, False), (48, 48, 12, True), (64, 70, 12, False), (40, 40, 24, False), (7, 5, 70, False)]
+
+
+def coarse(glx, orc, lx, ly, nc, two):
+    """Identity plus random terms of spectral radius 1/2, all shifts on."""
+    rng = np.random.default_rng(lx + 7 * ly + 31 * nc)
+    o = orc.CStencil.random(rng, lx, ly, nc, two, shifts=(0.1 + 0.05j, -0.05j, 0.1))
+    scale = 0.5 / np.sqrt(2.0 * nc * (13 if two else 5))
+    o.hopping *= scale
+    if two:
+        o.two_link *= scale
+    o.clover = (scale * o.clover.reshape(-1, nc, nc) + np.eye(nc)).reshape(-1)
+    g = glx.StencilNc(lx, ly, nc, o.clover, o.hopping, o.two_link if two else None, o.shift, o.eo_shift, o.dof_shift, 0)
+    b, x0 = (rng.standard_normal(o.n) + 1j * rng.standard_normal(o.n) for _ in range(2))
+    return o, glx.CStencilDev(g), b, x0
+
+
+def gcr_both(glx, resident, h, b, x0, **kw):
+    """(x, info) on the chip and with a launch per phase."""
+    out = []
+    for on in (True, False):
+        resident(on, 0)
+        dx = glx.DeviceArray(x0)
+        info = h.solve("gcr", dx, glx.DeviceArray(b), **kw)
+        out.append((dx.download(), info))
+    return out
+
+
+@pytest.mark.parametrize("lx,ly,nc,two", STENCILS)
+def test_gcr_on_the_general_stencil(glx, orc, resident, lx, ly, nc, two):
+    """The iterations of the launch-per-phase form (one apart where the norm
+    meets the tolerance within rounding) and its iterates; the residual by the
+    oracle's operator."""
+    print(f"case {lx} x {ly} nc={nc} two={two}", flush=True)
+    o, h, b, x0 = coarse(glx, orc, lx, ly, nc, two)
+    nb = np.linalg.norm(b)
+    (x, i), (xl, il) = gcr_both(glx, resident, h, b, x0, max_iter=400, eps=1e-10)
+    assert i.success and il.success and abs(i.iter - il.iter) <= 1 and i.ops_count == i.iter + 2
+    r = b - orc.cstencil_apply(o, x)
+    assert np.linalg.norm(r) <= 1.01e-10 * nb
+    # (entries of A x are sums of 13 nc products at most)
+    assert abs(np.sqrt(i.resSq) - np.linalg.norm(r)) <= 13 * nc * 1e-15 * nb
+    if lx * ly * nc > 60:  # (a small system is solved within so few)
+        for stop in (1, 2, 7):
+            (x, i), (xl, il) = gcr_both(glx, resident, h, b, x0, max_iter=stop, eps=1e-10)
+            assert (i.iter, i.success, i.ops_count) == (il.iter, il.success, il.ops_count)
+            assert relerr(x, xl) < 1e-12 and abs(i.resSq - il.resSq) <= 1e-10 * il.resSq
+
+
+def test_gcr_over_several_launches(glx, orc, resident):
+    """1.02 - (shift in x) converges by 1/1.02 per iteration: directions of one
+    launch, of several, and of more than the resident form holds, where a
+    launch per phase takes over."""
+    lx, ly = 1500, 2
+    n = lx * ly
+    hop = np.zeros((4, n, 1, 1), dtype=complex)
+    hop[0] = -1.0
+    g = glx.StencilNc(lx, ly, 1, np.full((n, 1, 1), 1.02 + 0j), hop, None)
+    h = glx.CStencilDev(g)
+    rng = np.random.default_rng(5)
+    b = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    nb = np.linalg.norm(b)
+
+    def residual(x):
+        x = x.reshape(ly, lx)
+        return np.linalg.norm(b - (1.02 * x - np.roll(x, -1, axis=1)).reshape(-1))
+
+    for stop, eps in ((64, 1e-10), (65, 1e-10), (130, 1e-10), (512, 1e-10), (513, 1e-10), (4000, 1e-6)):
+        (x, i), (xl, il) = gcr_both(glx, resident, h, b, np.zeros(n, dtype=complex), max_iter=stop, eps=eps)
+        print(stop, i.iter, il.iter, residual(x) / nb, flush=True)
+        assert i.success == il.success and abs(i.iter - il.iter) <= (0 if stop < 600 else 2)
+        assert abs(residual(x) - residual(xl)) <= (1e-8 if stop < 600 else 0.05) * residual(xl)
+        assert abs(np.sqrt(i.resSq) - residual(x)) <= 1e-13 * nb
+    assert i.success and i.iter > 520
+
+
+def test_gcr_waits_that_run_out(glx, orc, resident):
+    o, h, b, x0 = coarse(glx, orc, 32, 32, 8, False)
+    resident(True, 1)
+    dx = glx.DeviceArray(x0)
+    assert h.solve("gcr", dx, glx.DeviceArray(b), max_iter=400, eps=1e-10).success
+    assert np.linalg.norm(b - orc.cstencil_apply(o, dx.download())) <= 1.01e-10 * np.linalg.norm(b)
+
+
 def test_guess_stop_and_zero(glx, orc):
     """A guess that is nearly the solution, max_iter stops, b = 0."""
     lx, ly, m = 130, 70, 0.1
