@@ -310,6 +310,10 @@ __global__ __launch_bounds__(kBlock) void k_finalize(int nblk, Fin fin, RedWs ws
   if (gate_closed(gate)) return;
   finalize_body<NR, Fin>(nblk, fin, ws);
 }
+template <class Fin, class = void>
+struct wave_fin : std::false_type {};
+template <class Fin>
+struct wave_fin<Fin, std::void_t<decltype(Fin::kWave)>> : std::true_type {};
 template <int NR, class Fin>
 __device__ __forceinline__ void finalize_body(int nblk, const Fin& fin, RedWs ws) {
   __shared__ double sm[NR][kWaves];
@@ -330,8 +334,15 @@ __device__ __forceinline__ void finalize_body(int nblk, const Fin& fin, RedWs ws
       for (int k = 0; k < NR; k++) acc[k] += v[u][k];
     }
   }
-  block_sum<NR>(acc, sm);
-  if (threadIdx.x == 0) fin(acc);
+  // a finaliser with per-shift work declares kWave: the first wave runs it, a
+  // lane each for the shifts; the others are one thread's
+  if constexpr (wave_fin<Fin>::value) {
+    block_sum_all<NR>(acc, sm);
+    if (threadIdx.x < 64) fin(acc);
+  } else {
+    block_sum<NR>(acc, sm);
+    if (threadIdx.x == 0) fin(acc);
+  }
 }
 
 // Two adjacent elements as one aligned access (16 bytes for complex FP32):

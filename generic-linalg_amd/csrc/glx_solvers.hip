@@ -1060,30 +1060,44 @@ struct FinCgmInit {
 };
 // beta = -rsq / <p, Ap>, then the zeta / beta_s recurrences for active shifts
 // (generic_cg_m.cpp:106-122, :396-412).
+// Run by a wave, lane n on shift n: the shifts' recurrences are independent,
+// and one thread for them, waiting for each shift's loads in turn, took 5.1 us of the 66 us of a
+// batched iteration (16 systems, 12 shifts); 4.5 here.
 template <class T>
 struct FinCgmBeta {
+  static constexpr bool kWave = true;
   SolveState* s;
   __device__ void operator()(const double* v) const {
-    s->beta_prev = s->beta;
+    static_assert(kMaxShift <= 64, "a lane per shift");
+    const int n = threadIdx.x;
+    const bool on = n < s->n_rem;
+    const int m = on ? n : 0;
+    const c128 bc = s->beta, ac = s->alpha, zc = s->zeta[m], zpc = s->zeta_p[m];
+    const double rsq = s->rsq, shift = s->shifts[m];
     if constexpr (is_cx<T>::value) {
-      s->beta = cdiv(c128{-s->rsq, 0.0}, c128{v[0], v[1]});
-      const c128 b = s->beta, bp = s->beta_prev, a = s->alpha;
-      for (int n = 0; n < s->n_rem; n++) {
-        const c128 z = s->zeta[n], zp = s->zeta_p[n];
+      const c128 b = cdiv(c128{-rsq, 0.0}, c128{v[0], v[1]}), bp = bc, a = ac, z = zc, zp = zpc;
+      if (n == 0) {
+        s->beta_prev = bc;
+        s->beta = b;
+      }
+      if (on) {
         const c128 num = (z * zp) * bp;
-        const c128 sb = s->shifts[n] * b;
+        const c128 sb = shift * b;
         const c128 one_m{1.0 - sb.re, -sb.im};
         const c128 den = (b * a) * (zp - z) + (zp * bp) * one_m;
-        s->zeta[n] = cdiv(num, den);
+        const c128 zn = cdiv(num, den);
+        s->zeta[n] = zn;
         s->zeta_p[n] = z;
-        s->beta_s[n] = cdiv(b * s->zeta[n], s->zeta_p[n]);
+        s->beta_s[n] = cdiv(b * zn, z);
       }
     } else {
-      s->beta = {-s->rsq / v[0], 0.0};
-      const double b = s->beta.re, bp = s->beta_prev.re, a = s->alpha.re;
-      for (int n = 0; n < s->n_rem; n++) {
-        const double z = s->zeta[n].re, zp = s->zeta_p[n].re;
-        const double zn = (z * zp * bp) / (b * a * (zp - z) + zp * bp * (1.0 - s->shifts[n] * b));
+      const double b = -rsq / v[0], bp = bc.re, a = ac.re, z = zc.re, zp = zpc.re;
+      if (n == 0) {
+        s->beta_prev = bc;
+        s->beta = {b, 0.0};
+      }
+      if (on) {
+        const double zn = (z * zp * bp) / (b * a * (zp - z) + zp * bp * (1.0 - shift * b));
         s->zeta[n] = {zn, 0.0};
         s->zeta_p[n] = {z, 0.0};
         s->beta_s[n] = {b * zn / z, 0.0};
@@ -2918,7 +2932,7 @@ struct CgmWin {
   int flush;  // the window ended at the last finaliser: the next residual pass applies it
   long long upd_r, upd_x, upd_p;  // applied: residual terms, x_s and p_s updates (site-independent counts)
   c128 cp[kMaxShift], ax[kMaxShift];
-  c128 dp[kMaxShift][kWin], ex[kMaxShift][kWin];
+  c128 dp[kWin][kMaxShift], ex[kWin][kMaxShift];
 };
 
 // The window's terms for one site: r^(k0+1+j), j < wlen, from the ring.
@@ -2977,7 +2991,7 @@ struct PtCgmWindow {
     c128* lc = lds_c();
     for (int t = threadIdx.x; t < nx * kC; t += blockDim.x) {
       const int q = t / kC, c = t % kC;
-      lc[t] = c == 0 ? w->ax[q] : (c == 1 ? w->cp[q] : (c < 2 + kWin ? w->ex[q][c - 2] : w->dp[q][c - 2 - kWin]));
+      lc[t] = c == 0 ? w->ax[q] : (c == 1 ? w->cp[q] : (c < 2 + kWin ? w->ex[c - 2][q] : w->dp[c - 2 - kWin][q]));
     }
     T** lx = lds_x();
     T** lp = lds_p();
@@ -3081,7 +3095,7 @@ struct PtCgmFlushX {
       T xa = xtab[v][i] + w->ax[q] * ptab[v][i];
 #pragma unroll
       for (int j = 0; j < kWin; j++)
-        if (j < wlen) xa = xa + w->ex[q][j] * rj[j];
+        if (j < wlen) xa = xa + w->ex[j][q] * rj[j];
       xtab[v][i] = xa;
     }
   }
@@ -3089,87 +3103,146 @@ struct PtCgmFlushX {
 // FinCgmR with the window's coefficients: the x_s step of this iteration,
 // the check (permuting the coefficients with the shifts), alpha, alpha_s, the
 // p_s step, and whether the window ends here.
+// Run by a wave, lane q on shift q with its window coefficients (stored by
+// term, so that a term's load is one row of the lanes); only the permutation
+// of a check that finds converged shifts is one lane's.  One thread for all of
+// it took 10.9 us of the 66 us of a batched iteration (16 systems, 12 shifts);
+// 5.6 here.
 struct FinCgmRWin {
+  static constexpr bool kWave = true;
   SolveState* s;
   CgmWin* w;
-  __device__ static void swp(c128& a, c128& b) {
-    const c128 t = a;
+  template <class V>
+  __device__ static void swp(V& a, V& b) {
+    const V t = a;
     a = b;
     b = t;
   }
-  __device__ void operator()(const double* v) const {
-    const double rn = v[0];
-    const int k = s->k;
-    if (s->hist) s->hist[k] = sqrt(rn) / s->bsqrt;
-    const double tol = s->eps * s->bsqrt;
-    if (w->flush) {  // the previous window was applied by this iteration's window launch
-      w->flush = 0;
-      w->wlen = 0;
-      for (int q = 0; q < s->n_rem; q++) {
-        w->cp[q] = {1.0, 0.0};
-        w->ax[q] = {0.0, 0.0};
-        for (int j = 0; j < kWin; j++) w->dp[q][j] = w->ex[q][j] = {0.0, 0.0};
-      }
-    }
-    const int wl = w->wlen;
-    s->n_xupd = s->n_rem;
-    // x_s -= beta_s p_s (generic_cg_m.cpp:414-420) on the coefficients
-    for (int q = 0; q < s->n_rem; q++) {
-      const c128 b = s->beta_s[q];
-      w->ax[q] = w->ax[q] - b * w->cp[q];
-      for (int j = 0; j < wl; j++) w->ex[q][j] = w->ex[q][j] - b * w->dp[q][j];
-    }
-    if (k % s->resid_freq == 0) {
-      for (int n = 0; n < s->n_rem; n++) {
-        const double zabs = hypot(s->zeta[n].re, s->zeta[n].im);
-        if (zabs * sqrt(rn) < tol) {
-          s->n_rem--;
-          const int e = s->n_rem;
-          if (e != n) {
-            int t = s->mapping[e]; s->mapping[e] = s->mapping[n]; s->mapping[n] = t;
-            t = s->vec[e]; s->vec[e] = s->vec[n]; s->vec[n] = t;
-            swp(s->alpha_s[e], s->alpha_s[n]);
-            swp(s->beta_s[e], s->beta_s[n]);
-            swp(s->zeta[e], s->zeta[n]);
-            swp(s->zeta_p[e], s->zeta_p[n]);
-            const double d = s->shifts[e]; s->shifts[e] = s->shifts[n]; s->shifts[n] = d;
-            swp(w->cp[e], w->cp[n]);
-            swp(w->ax[e], w->ax[n]);
-            for (int j = 0; j < kWin; j++) {
-              swp(w->dp[e][j], w->dp[n][j]);
-              swp(w->ex[e][j], w->ex[n][j]);
-            }
-            n--;
+  // moves the converged shifts behind the active ones (generic_cg_m.cpp:429-470)
+  __device__ void drop(double rnorm, double tol) const {
+    for (int n = 0; n < s->n_rem; n++) {
+      if (hypot(s->zeta[n].re, s->zeta[n].im) * rnorm < tol) {
+        s->n_rem--;
+        const int e = s->n_rem;
+        if (e != n) {
+          swp(s->mapping[e], s->mapping[n]);
+          swp(s->vec[e], s->vec[n]);
+          swp(s->alpha_s[e], s->alpha_s[n]);
+          swp(s->beta_s[e], s->beta_s[n]);
+          swp(s->zeta[e], s->zeta[n]);
+          swp(s->zeta_p[e], s->zeta_p[n]);
+          swp(s->shifts[e], s->shifts[n]);
+          swp(w->cp[e], w->cp[n]);
+          swp(w->ax[e], w->ax[n]);
+          for (int j = 0; j < kWin; j++) {
+            swp(w->dp[j][e], w->dp[j][n]);
+            swp(w->ex[j][e], w->ex[j][n]);
           }
+          n--;
         }
       }
     }
-    const double z0 = hypot(s->zeta[0].re, s->zeta[0].im);
-    if ((s->worst_first && z0 * sqrt(rn) < tol) || s->n_rem == 0 || k == s->max_iter - 1) {
-      s->kfinal = k;
-      s->done = 1;
+  }
+  __device__ void operator()(const double* v) const {
+    static_assert(kMaxShift <= 64, "a lane per shift");
+    const int q = threadIdx.x;
+    const bool lead = q == 0;
+    const double rn = v[0], rnorm = sqrt(rn);
+    const int k = s->k, nx = s->n_rem;
+    const bool fresh = w->flush;  // the previous window was applied by this iteration's window launch
+    const int wl = fresh ? 0 : w->wlen;
+    if (lead && s->hist) s->hist[k] = rnorm / s->bsqrt;
+    const double tol = s->eps * s->bsqrt, rsq = s->rsq;
+    const bool check = k % s->resid_freq == 0;
+    const int last = s->max_iter - 1, worst = s->worst_first;
+    const c128 beta = s->beta;
+    bool on = q < nx;
+    int m = on ? q : 0;
+    c128 cp = fresh ? c128{1.0, 0.0} : w->cp[m], ax = fresh ? c128{0.0, 0.0} : w->ax[m];
+    c128 bs = s->beta_s[m], zt = s->zeta[m], zp = s->zeta_p[m];
+    c128 dp[kWin], ex[kWin];
+#pragma unroll
+    for (int j = 0; j < kWin; j++) {
+      dp[j] = ex[j] = {0.0, 0.0};
+      if (j < wl) {
+        dp[j] = w->dp[j][m];
+        ex[j] = w->ex[j][m];
+      }
+    }
+    // x_s -= beta_s p_s (generic_cg_m.cpp:414-420) on the coefficients
+    ax = ax - bs * cp;
+#pragma unroll
+    for (int j = 0; j < kWin; j++)
+      if (j < wl) ex[j] = ex[j] - bs * dp[j];
+    auto store = [&]() {
+      if (!on) return;
+      w->cp[q] = cp;
+      w->ax[q] = ax;
+#pragma unroll
+      for (int j = 0; j < kWin; j++) {
+        w->dp[j][q] = dp[j];
+        w->ex[j][q] = ex[j];
+      }
+    };
+    if (lead) {
+      if (fresh) w->flush = 0;
+      w->wlen = wl;
+      s->n_xupd = nx;
+    }
+    int nr = nx;
+    if (check && __ballot(on && hypot(zt.re, zt.im) * rnorm < tol)) {
+      store();
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
+      if (lead) drop(rnorm, tol);
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
+      nr = s->n_rem;
+      cp = w->cp[m];
+      ax = w->ax[m];
+      bs = s->beta_s[m];
+      zt = s->zeta[m];
+      zp = s->zeta_p[m];
+#pragma unroll
+      for (int j = 0; j < kWin; j++) {
+        dp[j] = w->dp[j][m];
+        ex[j] = w->ex[j][m];
+      }
+    }
+    const double z0 = hypot(readlane_d(zt.re, 0), readlane_d(zt.im, 0));
+    if ((worst && z0 * rnorm < tol) || nr == 0 || k == last) {
+      store();
+      if (lead) {
+        s->kfinal = k;
+        s->done = 1;
+      }
       return;
     }
-    const double al = rn / s->rsq;
-    s->alpha = {al, 0.0};
-    s->rsq = rn;
-    for (int n = 0; n < s->n_rem; n++)
-      s->alpha_s[n] = cdiv((s->alpha * s->zeta[n]) * s->beta_s[n], s->zeta_p[n] * s->beta);
-    // p_s = zeta_s r^(k+1) + alpha_s p_s (generic_cg_m.cpp:508-514) on the coefficients
-    for (int q = 0; q < s->n_rem; q++) {
-      const c128 a = s->alpha_s[q];
-      w->cp[q] = a * w->cp[q];
-      for (int j = 0; j < wl; j++) w->dp[q][j] = a * w->dp[q][j];
-      w->dp[q][wl] = s->zeta[q];
+    const c128 alpha{rn / rsq, 0.0};
+    if (q < nr) {
+      // p_s = zeta_s r^(k+1) + alpha_s p_s (generic_cg_m.cpp:508-514) on the coefficients
+      const c128 a = cdiv((alpha * zt) * bs, zp * beta);
+      s->alpha_s[q] = a;
+      cp = a * cp;
+#pragma unroll
+      for (int j = 0; j < kWin; j++) {
+        if (j < wl) dp[j] = a * dp[j];
+        if (j == wl) dp[j] = zt;
+      }
     }
-    w->wlen = wl + 1;
-    if (k % s->resid_freq == 0 || w->wlen == kWin) {
-      w->flush = 1;
-      w->upd_r += w->wlen;
-      w->upd_x += s->n_xupd;
-      w->upd_p += s->n_rem;
+    store();
+    if (lead) {
+      s->alpha = alpha;
+      s->rsq = rn;
+      w->wlen = wl + 1;
+      if (check || wl + 1 == kWin) {
+        w->flush = 1;
+        w->upd_r += wl + 1;
+        w->upd_x += nx;
+        w->upd_p += nr;
+      }
+      s->k = k + 1;
     }
-    s->k = k + 1;
   }
 };
 // Prologue of the batched D^dag D launch: p^(k+1) = r^(k+1) + alpha p^(k)
@@ -3433,8 +3506,15 @@ std::vector<SolveResult> cg_m_batch_impl(const std::vector<BatchSystem>& sys, in
   // submission pipeline, one pair of events around every phase launch of a
   // group; a slot's events are read after its group is waited for.  Groups
   // hold an even number of iterations: every group starts on p buffer 0.
-  const int group = 2 * ((std::max(1, opt.group) + 1) / 2);
+  // A replayed graph holds the same launches every time: where a whole number
+  // of check intervals fits, so that windows end at the same places of every
+  // group, the group is rounded up to that.
   const bool timing = time_phases && stats;
+  const bool graph = opt.use_graph && !timing;
+  int group = 2 * ((std::max(1, opt.group) + 1) / 2);
+  const long period = resid_freq % 2 ? 2L * resid_freq : resid_freq;
+  const bool aligned = period <= 2 * group;
+  if (graph && aligned) group = int((group + period - 1) / period * period);
   std::vector<hipEvent_t> tev;
   if (timing) {
     tev.resize(size_t(2) * group * 6);
@@ -3461,16 +3541,28 @@ std::vector<SolveResult> cg_m_batch_impl(const std::vector<BatchSystem>& sys, in
                        F_st.items.as<FinItem<FinCgmBeta<T>>>());
     GLX_CHECK_LAUNCH();
   };
+  // Windows end at the same iterations in every system that still runs, by the
+  // distance from the last check (FinCgmRWin), so the host knows which
+  // iterations have one to apply and leaves the launch out of the others: nine
+  // of ten at resid_freq = kWin.  A launch with nothing to apply took 4.6 us of
+  // an iteration's 50 (16 systems of 64^2 to 512^2, 12 shifts): 27.1 ms for the
+  // batch with it, 25.5 without.
+  const bool skips = !graph || aligned;
+  long n_enq = 0;
+  auto window_ended = [&](long k) { return k >= 0 && (k % resid_freq == 0 || (k % resid_freq) % kWin == 0); };
   // iteration at group position g: the window that ended at the last
-  // iteration (a launch that returns at once where none did), the residual
-  // pass and its finaliser, then D^dag D on p^(k+1) formed in the launch's
-  // prologue, and beta / zeta
+  // iteration, the residual pass and its finaliser, then D^dag D on p^(k+1)
+  // formed in the launch's prologue, and beta / zeta
   auto enq_iter = [&]() {
     const int c = t_iter & 1;
     tmark(1, 0);
-    hipLaunchKernelGGL((k_point_batch<PtCgmWindow<T>>), dim3(L_w.nblk_total), dim3(kBlock), 0, st,
-                       L_w.items.as<PtItem<PtCgmWindow<T>>>(), L_w.map());
-    GLX_CHECK_LAUNCH();
+    // (a graph's first group stands for all: there iteration 0 is any check)
+    if (!skips || window_ended(n_enq - 1) || (graph && n_enq == 0 && window_ended(resid_freq - 1))) {
+      hipLaunchKernelGGL((k_point_batch<PtCgmWindow<T>>), dim3(L_w.nblk_total), dim3(kBlock), 0, st,
+                         L_w.items.as<PtItem<PtCgmWindow<T>>>(), L_w.map());
+      GLX_CHECK_LAUNCH();
+    }
+    n_enq++;
     hipLaunchKernelGGL((k_point_batch<PtCgmRing<T>>), dim3(L_x.nblk_total), dim3(kBlock), 0, st,
                        L_x.items.as<PtItem<PtCgmRing<T>>>(), L_x.map());
     GLX_CHECK_LAUNCH();
@@ -3500,13 +3592,13 @@ std::vector<SolveResult> cg_m_batch_impl(const std::vector<BatchSystem>& sys, in
   launch_beta();
 
   hipGraphExec_t exec = nullptr;
-  if (opt.use_graph && !timing) {
-    hipGraph_t graph = nullptr;
+  if (graph) {
+    hipGraph_t g0 = nullptr;
     GLX_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     for (int g = 0; g < group; g++) enq_iter();
-    GLX_HIP(hipStreamEndCapture(st, &graph));
-    GLX_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    GLX_HIP(hipGraphDestroy(graph));
+    GLX_HIP(hipStreamEndCapture(st, &g0));
+    GLX_HIP(hipGraphInstantiate(&exec, g0, nullptr, nullptr, 0));
+    GLX_HIP(hipGraphDestroy(g0));
   }
   // control words of all systems: the first 16 bytes of each state, strided
   Mirror* pin = nullptr;

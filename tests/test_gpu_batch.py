@@ -72,6 +72,29 @@ def test_batched_multishift_matches_oracle(glx, orc, use_graph):
                 assert np.sqrt(info.resSqmrhs[k] / bn2) <= tol * 1.01 and np.sqrt(ro[k] / bn2) <= tol * 1.01
 
 
+@pytest.mark.parametrize("freq", [1, 3, 10, 11, 16, 25, 40])
+def test_batched_check_intervals(glx, orc, freq):
+    """Windows of shift updates that end at checks, after ten iterations, or
+    both, in groups that hold a whole number of intervals (even to 32, odd to 16) and in
+    groups that do not: replayed or launched one by one, the same bits, and the
+    residuals by the oracle's operator."""
+    shapes = [(64, 64), (128, 8)]
+    out = []
+    for use_graph in (True, False):
+        systems, ref = make_batch(glx, orc, shapes, 1)
+        infos = glx.dev_cg_m_batched(systems, SHIFTS, resid_freq_check=freq, max_iter=4000, eps=1e-10,
+                                     use_graph=use_graph)
+        out.append(([[x.download() for x in s[3]] for s in systems], [i.iter for i in infos]))
+    assert out[0][1] == out[1][1]
+    for (links, b, m, lx, ly), xs, ys, info in zip(ref, out[0][0], out[1][0], infos):
+        assert info.success
+        for k, (x, y) in enumerate(zip(xs, ys)):
+            assert np.array_equal(x, y)
+            r = b - orc.apply("staggered_normal", x, links, m, lx, ly) - SHIFTS[k] * x
+            assert np.linalg.norm(r) <= 2e-10 * np.linalg.norm(b)
+            assert abs(np.sqrt(info.resSqmrhs[k]) - np.linalg.norm(r)) <= 1e-12 * np.linalg.norm(b)
+
+
 def test_batched_equals_single_solves(glx, orc):
     """The batch gives each system what a solve of its own gives: the same
     iterations and ops_count, and solutions equal to the rounding of their
