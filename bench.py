@@ -14,8 +14,9 @@ time to solution in ms (lower is better).  The JSON line also carries the
 FP64 solves' times (the reference-order CG and the single-pass CG), the
 speed-ups, iteration counts, the solutions' relative errors against the FP64
 GPU solve and against the reference CPU solve of the same system, the
-roofline of the mixed solve's dominant kernel (the s-step launch) measured
-live with HIP events, the plain D and D^dag D stencils at this size, 2x this
+roofline of the s-step launch (the mixed iteration where a lattice does not
+fit the chip's registers; this one's solves are one resident launch each)
+measured live with HIP events, the plain D and D^dag D stencils at this size, 2x this
 size and 4096^2 (beyond the 256 MB last-level cache) as fractions of the HBM
 peak and of the streaming ceiling measured in the same run, the multishift
 batch with its per-phase roofline, and the reference CPU path timed on the
@@ -641,6 +642,9 @@ def main():
         tuned_ss = {"rows": args.sstep_rows}
     else:
         tuned_ss = glx.autotune_sstep(lat, reps=40)
+    # the mixed solve runs in one launch where the lattice fits 256 tiles of at
+    # most 60 x 80 sites and no launch form was asked for
+    resident = args.sstep_form is None and -(-L // 60) * -(-L // 80) <= 256
     d_b = glx.DeviceArray(b)
     d_x = glx.DeviceArray(np.zeros_like(b))
     d_x64 = glx.DeviceArray(np.zeros_like(b))
@@ -705,12 +709,12 @@ def main():
     xmx = d_x.download()
     err_vs_fp64 = float(np.linalg.norm(xmx - x64) / np.linalg.norm(x64))
 
-    # live roofline of the mixed solve's dominant kernel: the s-step launch
+    # live roofline of the mixed iteration in launches: the s-step launch
     # (two CG iterations: p, r, x from the previous basis, then A p, A^2 p,
     # A r and twelve FP64 partial sums), HIP events around back-to-back
     # launches on its own stream; the one-iteration kernel beside it
     it_ms, it_bps = glx.time_cg_kernel(lat, mass, prec=2 + link_prec, reps=200)
-    ss_form = glx.get_sstep_form_for(L, L)  # the form the timed launch (and the solves) took
+    ss_form = glx.get_sstep_form_for(L, L)  # the form the timed launch takes
     it1_ms, it1_bps = glx.time_cg_kernel(lat, mass, prec=link_prec, reps=200)
     it64_ms, it64_bps = glx.time_cg_kernel(lat, mass, prec=0, reps=200)
     it_gbs = it_bps * V / (it_ms * 1e-3) / 1e9
@@ -781,7 +785,8 @@ def main():
         "speedup_vs_fp64": round(ms64 / msmx, 3),
         "speedup_basis": "plain FP64 GPU CG in the reference's order of operations (glx_dev_solve)",
         "speedup_vs_fp64_fused": round(msfu / msmx, 3),
-        "mixed_form": (("s-step, two CG iterations per launch, "
+        "mixed_form": ("one launch per solve, the system in registers" if resident else
+                       ("s-step, two CG iterations per launch, "
                         + ("wave strips (form 1)" if glx.get_sstep_form_for(L, L) == 1
                            else f"{tuned_ss['rows']} rows per block (form 0)")
                         + f" ({'set' if args.sstep_rows > 0 else 'autotuned'})")
