@@ -2560,8 +2560,9 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, void* x, const 
   RsSolve so{};
   so.x = static_cast<c128*>(x);
   so.b = static_cast<const c128*>(b);
-  so.u64 = o.u64;
-  so.lk = RsLinks{o.u64, nullptr, LINKS_F64};
+  // (a lattice carries links for every operator kind; the free Laplacian's are unit)
+  so.u64 = op_links(o.kind) ? o.u64 : nullptr;
+  so.lk = RsLinks{so.u64, nullptr, LINKS_F64};
   if (form == RSF_MIXED)
     so.lk = mo.link_prec == LINKS_F16 ? RsLinks{o.u16, o.sc16, LINKS_F16} : RsLinks{o.u32, nullptr, LINKS_F32};
   if (op_links(o.kind) && (!so.u64 || !so.lk.u || (so.lk.prec == LINKS_F16 && !so.lk.sc)))

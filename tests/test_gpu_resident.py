@@ -151,6 +151,24 @@ def test_one_hop_bicgstab(glx, orc, lx, ly, op, mass):
     assert abs(np.sqrt(ig.resSq) - np.linalg.norm(r)) <= 1e-12 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("solver", ["cg", "bicgstab"])
+@pytest.mark.parametrize("op", ["laplace", "laplace_real", "laplace_u1"])
+def test_laplacians_on_a_lattice_with_links(glx, orc, solver, op):
+    """The free Laplacians take only their dimensions from a lattice, whose
+    links are far from unit here; laplace_u1 takes both.  The residual is the
+    oracle's operator's, as reported."""
+    lx, ly, m = 61, 23, 0.05
+    links, bc, br = lattice_inputs(orc, lx, ly, beta=2.0, seed=77)
+    b = br if op == "laplace_real" else bc
+    dx = glx.DeviceArray(np.zeros_like(b))
+    info = glx.dev_solve(solver, glx.Lattice(links, lx, ly), op, m, dx, glx.DeviceArray(b), max_iter=5000, eps=1e-10)
+    r = b - orc.apply(op, dx.download(), links, m, lx, ly)
+    nb = np.linalg.norm(b)
+    # (BiCGStab's iterated residual may drift from the true one)
+    assert info.success and np.linalg.norm(r) <= (1e-9 if solver == "bicgstab" else 1.001e-10) * nb
+    assert abs(np.sqrt(info.resSq) - np.linalg.norm(r)) <= 1e-12 * nb
+
+
 @pytest.mark.parametrize("lx,ly,n_shift,freq", [(4, 8, 1, 1), (4, 8, 16, 10), (60, 9, 5, 3), (61, 23, 16, 10),
                                                 (130, 70, 2, 7), (200, 144, 12, 10)])
 def test_multishift_matches_oracle(glx, orc, lx, ly, n_shift, freq):
