@@ -33,6 +33,7 @@
 
 #include "glx_cstencil.h"
 #include "glx_restile.h"
+#include "glx_rgwalk.h"
 
 namespace glx {
 
@@ -59,14 +60,14 @@ struct RsGcr {
   RsOut* out;
 };
 
-__host__ __device__ constexpr int rg_pitch(int nc) { return nc | 1; }  // colours of a staged site, an odd count for the banks
+static_assert(kRgWaves == kRsWaves, "the walk's waves");
 __host__ __device__ constexpr int rg_words(int k0) { return 2 * (k0 + kRgDirs + 1); }
 
 template <int M>
 __global__ __launch_bounds__(kRsThreads) void k_rs_gcr(RsGcr g) {
   constexpr int NW = kRsWaves, EW = 64 * M;           // entries a block may own
   constexpr int Q = (12 * EW + kRsThreads - 1) / kRsThreads;  // staged values per thread
-  constexpr int KF = M == 1 ? 24 : (M == 2 ? 8 : 4);  // coefficients kept per entry
+  constexpr int KF = rg_kept(M);
   const int nc = g.st.nc, n = g.st.lx * g.st.ly * nc, pitch = rg_pitch(nc);
   extern __shared__ c128 lds[];
   c128* stage = lds;                                  // [nt][sites][pitch]
@@ -109,8 +110,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_gcr(RsGcr g) {
     }
   }
   // the wave's columns f of all terms': f0 to f1, the first KF kept
-  const int nf = g.nt * nc, wf = (nf + NW - 1) / NW;
-  const int f0 = min(wave * wf, nf - 1), f1 = min(wave * wf + wf, nf), t0 = f0 / nc;
+  const int nf = g.nt * nc, wf = rg_share(nf);
+  const int f0 = rg_first(nf, wave), f1 = rg_end(nf, wave);
   const c128* __restrict__ coef = g.st.coef + i0 + lane;
   c128 kept[KF][M];
 #pragma unroll
@@ -147,17 +148,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_gcr(RsGcr g) {
   auto apply_staged = [&](c128 (&av)[M]) {
 #pragma unroll
     for (int m = 0; m < M; m++) av[m] = z;
-    int at = t0 * tspan + f0 - t0 * nc, c = f0 - t0 * nc;
-    const int last = g.nt * tspan - (g.sites - 1) * pitch - 1;  // (where a zero coefficient may point)
-    auto step = [&]() {
-      c++;
-      at++;
-      if (c == nc) {
-        at += tspan - nc;
-        c = 0;
-      }
-      at = min(at, last);
-    };
+    RgWalk w(g.nt, nc, g.sites, f0);
     // four at a time without a branch: columns beyond f1 have zeros
 #pragma unroll
     for (int q0 = 0; q0 < KF; q0 += 4) {
@@ -165,8 +156,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_gcr(RsGcr g) {
 #pragma unroll
         for (int q = q0; q < q0 + 4; q++) {
 #pragma unroll
-          for (int m = 0; m < M; m++) av[m] = av[m] + kept[q][m] * stage[at + own[m]];
-          step();
+          for (int m = 0; m < M; m++) av[m] = av[m] + kept[q][m] * stage[w.at + own[m]];
+          w.step();
         }
       }
     }
@@ -174,8 +165,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_gcr(RsGcr g) {
     for (int f = f0 + KF; f < f1; f++) {
 #pragma unroll
       for (int m = 0; m < M; m++)
-        if (has[m]) av[m] = av[m] + coef[size_t(f) * n + 64 * m] * stage[at + own[m]];
-      step();
+        if (has[m]) av[m] = av[m] + coef[size_t(f) * n + 64 * m] * stage[w.at + own[m]];
+      w.step();
     }
     meet(av, [&](int e, c128 a) {
       if (e >= ne) return z;
