@@ -47,6 +47,9 @@ class NoAllocScope {
   void* take(size_t bytes);
   hipStream_t stream() const { return stream_; }
   size_t used() const { return used_; }
+  // Gives back what was taken since used() was `mark`, once the stream has
+  // drained of its users.
+  void rewind(size_t mark) { used_ = mark; }
 
  private:
   char* base_;
@@ -56,6 +59,22 @@ class NoAllocScope {
 };
 // the calling thread's scope, or nullptr
 NoAllocScope* noalloc_scope();
+
+// Gives the calling thread's scope, if it has one, back what a part of a solve
+// took from it; that part's buffers are out of use by then.
+class ScopeRewind {
+ public:
+  ScopeRewind() : s_(noalloc_scope()), mark_(s_ ? s_->used() : 0) {}
+  ~ScopeRewind() {
+    if (s_) s_->rewind(mark_);
+  }
+  ScopeRewind(const ScopeRewind&) = delete;
+  ScopeRewind& operator=(const ScopeRewind&) = delete;
+
+ private:
+  NoAllocScope* s_;
+  size_t mark_;
+};
 
 // RAII device buffer from the pool (or from the thread's NoAllocScope).
 class DevBuf {

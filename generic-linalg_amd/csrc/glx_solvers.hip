@@ -2582,6 +2582,10 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, void* x, const 
     so.fx = so.fy_odd = -1.0;
   }
   const int words = cplx && form != RSF_MIXED ? rs_words<c128>() : 1;
+  // (an allocation-free caller's region holds either these, 36 MiB at
+  // 1020 x 1020, or the 104 MiB of the s-step form that repeats a solve which
+  // gave up, not both)
+  ScopeRewind rewind;
   DevBuf ex(size_t(rs_exchange_words(g, words, hop ? 1 : 2)) * 8);
   DevBuf out(sizeof(RsOut)), hist(opt.want_hist ? size_t(opt.max_iter) * sizeof(double) : 0);
   so.lines = ex.as<unsigned long long>();

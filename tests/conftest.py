@@ -36,6 +36,13 @@ def orc():
 
 
 @pytest.fixture
+def resident(glx):
+    """glx.set_resident, with its defaults back afterwards."""
+    yield glx.set_resident
+    glx.set_resident(True, 0)
+
+
+@pytest.fixture
 def rows_reset(glx, monkeypatch):
     """Launch-shape table entries a test sets through glx.set_normal_rows are
     removed afterwards and the default goes back to -1 (by block count), so

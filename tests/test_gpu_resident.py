@@ -20,12 +20,6 @@ SIZES = [(4, 8), (5, 9), (60, 8), (61, 23), (64, 16), (130, 70), (97, 301), (330
 LARGE = [(300, 512), (512, 400), (700, 512), (780, 780), (1000, 900)]
 
 
-@pytest.fixture
-def resident(glx):
-    yield glx.set_resident
-    glx.set_resident(True, 0)
-
-
 def system(glx, orc, lx, ly, beta=6.25):
     links, b, _ = lattice_inputs(orc, lx, ly, beta=beta, seed=1000 + lx + 3 * ly)
     return links, b, glx.Lattice(links, lx, ly), glx.DeviceArray(b)

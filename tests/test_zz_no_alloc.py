@@ -31,9 +31,14 @@ def _same(xa, ia, xb, ib):
     assert np.array_equal(xa, xb), relerr(xb, xa)
 
 
-@pytest.mark.parametrize("sstep", [2, 1])
-def test_noalloc_equals_mixed_two_calls(glx, orc, sstep):
+@pytest.mark.parametrize("sstep,on,spins", [(2, True, 0), (2, False, 0), (2, True, 1), (1, True, 0)],
+                         ids=["resident", "sstep", "given_up", "one_iteration"])
+def test_noalloc_equals_mixed_two_calls(glx, orc, resident, sstep, on, spins):
+    """The resident launch; the s-step launches, whose buffers take 104 of the
+    array's 112 MiB; those after a resident launch that gave up (a single poll
+    per wait), whose own 36 MiB have to be free again; one iteration per launch."""
     glx.set_sstep(sstep)
+    resident(on, spins)
     try:
         for (lx, ly, mass, beta) in [(1024, 1024, 0.02, 4.0), (256, 128, 0.05, 6.25)]:
             links, bc, _ = lattice_inputs(orc, lx, ly, beta=beta, seed=900 + lx + ly)
