@@ -26,12 +26,17 @@ struct ArgError : std::runtime_error {
   explicit ArgError(const std::string& s) : std::runtime_error(s) {}
 };
 
-#define GLX_HIP(call)                                                                          \
-  do {                                                                                         \
-    hipError_t e_ = (call);                                                                    \
-    if (e_ != hipSuccess)                                                                      \
-      throw ::glx::HipError(std::string(#call) + ": " + hipGetErrorString(e_) + " (" __FILE__ \
-                            ":" + std::to_string(__LINE__) + ")");                             \
+// (the runtime keeps a failed call's error for hipGetLastError, also past calls
+// that succeed: an error that is reported by the exception is taken off there,
+// or the check of a later launch would report it again)
+#define GLX_HIP(call)                                                                           \
+  do {                                                                                          \
+    hipError_t e_ = (call);                                                                     \
+    if (e_ != hipSuccess) {                                                                     \
+      (void)hipGetLastError();                                                                  \
+      throw ::glx::HipError(std::string(#call) + ": " + hipGetErrorString(e_) + " (" __FILE__  \
+                            ":" + std::to_string(__LINE__) + ")");                              \
+    }                                                                                           \
   } while (0)
 
 #define GLX_CHECK_LAUNCH() GLX_HIP(hipGetLastError())

@@ -149,6 +149,7 @@ void* DevicePool::alloc(size_t bytes) {
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, bytes);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // (not the next launch's)
     trim();
     GLX_HIP(hipMalloc(&p, bytes));
   }
