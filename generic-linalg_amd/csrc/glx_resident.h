@@ -262,6 +262,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
   A a;
   if constexpr (M == RS_REF) a = zero_of<T>();
   else a = Re(0);
+  double al = 0.0;  // (single-pass) alpha in FP64
   Re be = Re(0);
   double rsq = 0.0, maxrr = 0.0, bsqrt = 0.0, resSq = 0.0;
   const int kmax = so.max_iter - 1;
@@ -371,10 +372,16 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
       be = Re(rn / rsq);
       rsq = rn;
     } else {
-      // <p, Ap>, |Ap|^2, <Ap, r>, |r|^2 (real parts; A is Hermitian)
+      // <p, Ap>, |Ap|^2, <Ap, r>, |r|^2: real parts.  A is Hermitian for any
+      // stored links (K is anti-Hermitian in them), so the exact <p, Ap> and
+      // alpha are real, and imaginary parts of the sums are rounding alone:
+      // the real quotient's error against extended precision is no larger than
+      // that of rr / complex <p, Ap> (FP32 p: 1.4e-9 and 1.8e-9 at 64^2, 5.5e-11
+      // and 2.5e-10 at 512^2; FP64 equal).  alpha lies in scalar registers: in
+      // vector ones it spilled at ten rows.
       // (a zero residual ends the solve: no step)
       rsq = v1[3];
-      const double al = rsq == 0.0 ? 0.0 : rsq / v1[0];
+      al = rsq == 0.0 ? 0.0 : readlane_d(rsq / v1[0], 0);
       double rn = rsq - 2.0 * al * v1[2] + al * al * v1[1];
       if (!(rn > 0.0)) rn = 0.0;
       if (rn > maxrr) maxrr = rn;
@@ -389,10 +396,11 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
     k++;
     }
 
-    // ---- the solution to memory, for the true residual
+    // ---- the solution to memory, for the true residual: the last step and, in
+    // mixed precision, the sum with the FP64 solution in FP64
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      if constexpr (M != RS_REF) xref(j) = rs_axpy(a, p[j], xref(j));
+      if constexpr (M == RS_ONE) xref(j) = rs_axpy(a, p[j], xref(j));
       int y = yw;
       asm volatile("" : "+s"(y));
       const int i = at(y + j);
@@ -400,7 +408,11 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_cg(RsGeom g, RsSolve so) {
         unsigned long long* q = reinterpret_cast<unsigned long long*>(so.x + i);
         c128 v;
         cvt(v, xref(j));
-        if constexpr (M == RS_MIXED) v = rs_read<c128>(q) + v;
+        if constexpr (M == RS_MIXED) {
+          c128 pj;
+          cvt(pj, p[j]);
+          v = rs_read<c128>(q) + rs_axpy(al, pj, v);
+        }
         rs_put<c128>(q, v);
       }
       if constexpr (M == RS_MIXED) xref(j) = zero_of<T>();

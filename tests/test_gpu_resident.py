@@ -66,6 +66,28 @@ def test_mixed_matches_oracle(glx, orc, lx, ly, links_prec):
     assert np.linalg.norm(x - xs) <= 1.01e-10 * np.linalg.norm(b) / m**2
 
 
+@pytest.mark.parametrize("on", [True, False], ids=["resident", "launches"])
+@pytest.mark.parametrize("lx,ly", [(61, 23), (330, 222), (780, 780)])
+def test_mixed_adds_to_the_solution_in_fp64(glx, orc, resident, lx, ly, on):
+    """A reliable update is x64 += x32 + alpha p in FP64 with alpha in FP64.
+    After one iteration x32 = 0 and p = b, exact in FP32 here, so every
+    entry of x / b is the one alpha to a few FP64 roundings (in FP32 they
+    would differ by 1e-7); alpha itself is the FP64 one to the FP32 hops'
+    rounding."""
+    resident(on)
+    m = 0.1
+    links, b, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=1000 + lx + 3 * ly)
+    b = b.astype(np.complex64).astype(np.complex128)
+    dx = glx.DeviceArray(np.zeros_like(b))
+    info = glx.dev_cg_mixed(glx.Lattice(links, lx, ly), "staggered_normal", m, dx, glx.DeviceArray(b), max_iter=1)
+    assert info.iter == 1 and info.reliable_updates == 1
+    alpha = dx.download() / b
+    want = np.vdot(b, b).real / np.vdot(b, orc.apply("staggered_normal", b, links, m, lx, ly)).real
+    # (a complex product and quotient: 4 roundings each)
+    assert np.max(np.abs(alpha - alpha[0])) <= 16 * np.finfo(float).eps * abs(alpha[0])
+    assert abs(alpha[0] - want) <= 1e-6 * want
+
+
 @pytest.mark.parametrize("lx,ly", LARGE)
 def test_large_tiles_match_the_launch_per_iteration(glx, orc, resident, lx, ly):
     """Both run the same algorithm; their solutions stop at the same residual
