@@ -1380,6 +1380,13 @@ int glx_set_tuning(int group, int use_graph) {
 int glx_set_resident(int on, int spins) {
   return guarded([&] { set_resident(on, spins); });
 }
+int glx_get_resident_counts(long long* ran, long long* gave_up) {
+  return guarded([&] {
+    const RsCounts c = resident_counts();
+    if (ran) *ran = c.ran;
+    if (gave_up) *gave_up = c.gave_up;
+  });
+}
 int glx_set_sstep(int s, int rows) {
   return guarded([&] { set_sstep(s, rows); });
 }

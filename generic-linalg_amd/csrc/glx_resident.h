@@ -438,6 +438,13 @@ void set_resident(int on, int spins);
 bool resident_on();
 int rs_cus();  // CUs of the current device
 int resident_spins();
+// Solves that ran resident and solves whose resident launch gave up, of the
+// process so far.
+struct RsCounts {
+  long long ran, gave_up;
+};
+RsCounts resident_counts();
+void rs_count(bool gave_up);
 
 // The tiling a system would run resident with on the current device, for an
 // operator that reaches `halo` sites and kernels of at most most_rows rows per

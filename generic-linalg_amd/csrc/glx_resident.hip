@@ -14,6 +14,7 @@ std::atomic<int> g_on{1};
 // a poll takes about a microsecond: a second in all before a wait gives up
 constexpr int kSpins = 1 << 20;
 std::atomic<int> g_spins{kSpins};
+std::atomic<long long> g_ran{0}, g_gave_up{0};
 
 constexpr int kMaxDevices = 64;
 int current_device() {
@@ -90,6 +91,8 @@ void set_resident(int on, int spins) {
 int rs_cus() { return device_cus(current_device()); }
 bool resident_on() { return g_on.load() != 0; }
 int resident_spins() { return g_spins.load(); }
+RsCounts resident_counts() { return {g_ran.load(), g_gave_up.load()}; }
+void rs_count(bool gave_up) { (gave_up ? g_gave_up : g_ran)++; }
 
 bool rs_plan(int lx, int ly, int halo, int most_rows, RsGeom& g) {
   if (lx < 2 * halo || long(lx) * ly > (1L << 24)) return false;

@@ -2602,6 +2602,7 @@ static std::optional<SolveResult> rs_solve(const DevOperator& o, void* x, const 
     GLX_HIP(hipMemcpyAsync(&h, so.out, sizeof(h), hipMemcpyDeviceToHost, st));
     GLX_HIP(hipStreamSynchronize(st));
   }
+  rs_count(h.err || !h.done);
   if (h.err || !h.done) return std::nullopt;
   SolveResult res;
   res.iter = h.kfinal + 1;
@@ -2676,6 +2677,7 @@ static std::optional<SolveResult> rs_solve_cg_m(const DevOperator& o, void* cons
     GLX_HIP(hipMemcpyAsync(r.resSqmrhs.data(), res.get(), sizeof(double) * n_shift, hipMemcpyDeviceToHost, st));
     GLX_HIP(hipStreamSynchronize(st));
   }
+  rs_count(h.err || !h.done);
   if (h.err || !h.done) return std::nullopt;
   r.name = "CG-M";
   r.success = h.kfinal != opt.max_iter - 1;
@@ -2740,9 +2742,13 @@ static std::optional<SolveResult> rs_solve_gcr(const DevOperator& o, void* x, co
       GLX_HIP(hipMemcpyAsync(&h, g.out, sizeof(h), hipMemcpyDeviceToHost, st));
       GLX_HIP(hipStreamSynchronize(st));
     }
-    if (h.err) return std::nullopt;
+    if (h.err) {
+      rs_count(true);
+      return std::nullopt;
+    }
     if (c == 0) g.bsqrt = h.bsqrt;
   }
+  rs_count(false);
   if (!h.done) {
     GLX_HIP(hipMemcpyAsync(x, g.xs, vb, hipMemcpyDeviceToDevice, st));
     s.k = kRgDirs * kRgChunks;

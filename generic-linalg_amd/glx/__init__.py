@@ -211,6 +211,9 @@ def lib():
         if hasattr(L, "glx_set_resident"):  # absent from builds that predate it
             L.glx_set_resident.restype = i
             L.glx_set_resident.argtypes = [i, i]
+        if hasattr(L, "glx_get_resident_counts"):
+            L.glx_get_resident_counts.restype = i
+            L.glx_get_resident_counts.argtypes = [C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
         L.glx_set_sstep.restype = i
         L.glx_set_sstep.argtypes = [i, i]
         L.glx_get_sstep.restype = i
@@ -664,6 +667,13 @@ def set_resident(on: bool = True, spins: int = 0):
     and how often a block polls for another's value before the launch gives
     up and the solve runs with a launch per iteration (0: the default)."""
     _check(lib().glx_set_resident(int(on), int(spins)), "glx_set_resident")
+
+
+def resident_counts():
+    """(solves that ran resident, solves whose resident launch gave up) so far."""
+    ran, gave_up = C.c_longlong(), C.c_longlong()
+    _check(lib().glx_get_resident_counts(C.byref(ran), C.byref(gave_up)), "glx_get_resident_counts")
+    return ran.value, gave_up.value
 
 
 def set_sstep(s: int = 2, rows: int = 0):

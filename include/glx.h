@@ -456,6 +456,11 @@ int glx_set_tuning(int group, int use_graph);
  * glx_set_sstep_form (other than their defaults) keeps the mixed solver on
  * that form. */
 int glx_set_resident(int on, int spins);
+/* How many solves of this process ran resident so far, and how many had a
+ * resident launch that gave up and were repeated with a launch per iteration
+ * (each costs about a second at the default spins: another process holds the
+ * chip, for instance).  Either pointer may be NULL. */
+int glx_get_resident_counts(long long* ran, long long* gave_up);
 /* Iterations per launch of the mixed-precision CG on D^dag D (no reference
  * counterpart): s = 2 (default) runs two CG iterations per launch in s-step
  * form (basis p, Ap, A^2 p, r, Ar and its Gram matrix, FP32 vectors, FP64

@@ -3,11 +3,21 @@ by the oracle, bit-identical to the reference's own generators) and the
 envelopes the GPU results are held to: what the oracle's own results do
 under 1-ulp perturbations of the input and other valid reduction orders."""
 import concurrent.futures as cf
+import contextlib
 import os
 
 import numpy as np
 
 WORKERS = min(8, os.cpu_count() or 4)
+
+
+@contextlib.contextmanager
+def resident_solves(glx, n, gave_up=0):
+    """The block's solves: n run resident, gave_up give up and are repeated."""
+    r0, g0 = glx.resident_counts()
+    yield
+    r1, g1 = glx.resident_counts()
+    assert (r1 - r0, g1 - g0) == (n, gave_up), (r1 - r0, g1 - g0, n, gave_up)
 
 
 def pmap(fn, items):

@@ -3,13 +3,14 @@ the reference's order, single-pass and mixed precision, and the even/odd
 solves, at the sizes where the tiling can go wrong -- strips of one column
 count and of two, 60 and 61 columns, bands whose last one shares rows with the
 band before it, every number of rows per wave, lattices of one tile, odd sizes
--- and the way back to a launch per iteration when a wait runs out."""
+-- and the way back to a launch per iteration when a wait runs out.  Each test
+also counts the solves that ran resident and those that gave up."""
 import threading
 
 import numpy as np
 import pytest
 
-from helpers import ENVELOPE, bicgstab_envelope, eo_envelope, lattice_inputs, relerr
+from helpers import ENVELOPE, bicgstab_envelope, eo_envelope, lattice_inputs, relerr, resident_solves
 
 pytestmark = pytest.mark.gpu
 
@@ -36,13 +37,15 @@ def test_cg_matches_oracle(glx, orc, lx, ly):
     kw = dict(links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-10)
     runs = [orc.solve("cg", "staggered_normal", b, None, reductions=red, **kw) for red in ("serial", "extended")]
     dx = glx.DeviceArray(np.zeros_like(b))
-    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+    with resident_solves(glx, 1):
+        ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
     assert ig.iter in [io.iter for _, io in runs]
     xo, io = next(r for r in runs if r[1].iter == ig.iter)
     assert (ig.ops_count, ig.success) == (io.ops_count, io.success)
     assert relerr(dx.download(), xo) < 1e-11
     dx.upload(np.zeros_like(b))
-    jg = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db, max_iter=5000)
+    with resident_solves(glx, 1):
+        jg = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db, max_iter=5000)
     assert abs(jg.iter - io.iter) <= 2 and jg.success
     r = b - orc.apply("staggered_normal", dx.download(), links, m, lx, ly)
     # (A x is rounded to 4 u |x|, and |x| <= |b| / m^2 = 100 |b|: 1e-13 |b|)
@@ -57,7 +60,8 @@ def test_mixed_matches_oracle(glx, orc, lx, ly, links_prec):
     links, b, lat, db = system(glx, orc, lx, ly)
     xs, _ = orc.solve("cg", "staggered_normal", b, None, links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-13)
     dx = glx.DeviceArray(np.zeros_like(b))
-    info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, link_prec=links_prec)
+    with resident_solves(glx, 1):
+        info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, link_prec=links_prec)
     x = dx.download()
     r = b - orc.apply("staggered_normal", x, links, m, lx, ly)
     assert info.success and info.reliable_updates > 0
@@ -79,7 +83,8 @@ def test_mixed_adds_to_the_solution_in_fp64(glx, orc, resident, lx, ly, on):
     links, b, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=1000 + lx + 3 * ly)
     b = b.astype(np.complex64).astype(np.complex128)
     dx = glx.DeviceArray(np.zeros_like(b))
-    info = glx.dev_cg_mixed(glx.Lattice(links, lx, ly), "staggered_normal", m, dx, glx.DeviceArray(b), max_iter=1)
+    with resident_solves(glx, int(on)):
+        info = glx.dev_cg_mixed(glx.Lattice(links, lx, ly), "staggered_normal", m, dx, glx.DeviceArray(b), max_iter=1)
     assert info.iter == 1 and info.reliable_updates == 1
     alpha = dx.download() / b
     want = np.vdot(b, b).real / np.vdot(b, orc.apply("staggered_normal", b, links, m, lx, ly)).real
@@ -99,12 +104,13 @@ def test_large_tiles_match_the_launch_per_iteration(glx, orc, resident, lx, ly):
         resident(on)
         for name in ("cg", "fused", "mixed"):
             dx = glx.DeviceArray(np.zeros_like(b))
-            if name == "cg":
-                info = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db)
-            elif name == "fused":
-                info = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db)
-            else:
-                info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
+            with resident_solves(glx, int(on)):
+                if name == "cg":
+                    info = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db)
+                elif name == "fused":
+                    info = glx.dev_cg_fused(lat, "staggered_normal", m, dx, db)
+                else:
+                    info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
             assert info.success
             out[name, on] = (info, dx.download())
     for name in ("cg", "fused", "mixed"):
@@ -120,7 +126,8 @@ def test_even_odd(glx, orc, lx, ly, method):
     links, b, lat, db = system(glx, orc, lx, ly)
     xs, err = eo_envelope(orc, b, links, m, lx, ly)
     dx = glx.DeviceArray(np.zeros_like(b))
-    info, _ = glx.dev_solve_staggered_eo(lat, m, dx, db, method)
+    with resident_solves(glx, 1):
+        info, _ = glx.dev_solve_staggered_eo(lat, m, dx, db, method)
     assert info.success
     assert relerr(dx.download(), xs) <= ENVELOPE * err
 
@@ -139,7 +146,8 @@ def test_one_hop_cg_matches_oracle(glx, orc, lx, ly, op):
     kw = dict(links=links, mass=0.05, lx=lx, ly=ly, max_iter=5000)
     xs, _ = orc.solve("cg", op, b, None, eps=1e-13, **kw)
     xo, io = orc.solve("cg", op, b, None, eps=1e-10, **kw)
-    xg, ig = glx.minv_vector_cg(op, b, eps=1e-10, **kw)
+    with resident_solves(glx, 1):
+        xg, ig = glx.minv_vector_cg(op, b, eps=1e-10, **kw)
     assert ig.success and abs(ig.iter - io.iter) <= 1 and ig.ops_count == ig.iter + 2
     if ig.iter == io.iter:
         assert relerr(xg, xo) < 1e-11
@@ -157,7 +165,8 @@ def test_one_hop_bicgstab(glx, orc, lx, ly, op, mass):
     reported."""
     links, b, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=600 + lx + ly)
     kw = dict(links=links, mass=mass, lx=lx, ly=ly, max_iter=5000)
-    xg, ig = glx.minv_vector_bicgstab(op, b, eps=1e-10, **kw)
+    with resident_solves(glx, 1):
+        xg, ig = glx.minv_vector_bicgstab(op, b, eps=1e-10, **kw)
     _, _, its, _ = bicgstab_envelope(orc, op, b, dict(kw, eps=1e-10))
     width = max(2, its.max() - its.min())
     assert ig.success and ig.ops_count == 2 * ig.iter + 2
@@ -177,7 +186,9 @@ def test_laplacians_on_a_lattice_with_links(glx, orc, solver, op):
     links, bc, br = lattice_inputs(orc, lx, ly, beta=2.0, seed=77)
     b = br if op == "laplace_real" else bc
     dx = glx.DeviceArray(np.zeros_like(b))
-    info = glx.dev_solve(solver, glx.Lattice(links, lx, ly), op, m, dx, glx.DeviceArray(b), max_iter=5000, eps=1e-10)
+    # (BiCGStab on the real Laplacian has no resident kernel)
+    with resident_solves(glx, 0 if (solver, op) == ("bicgstab", "laplace_real") else 1):
+        info = glx.dev_solve(solver, glx.Lattice(links, lx, ly), op, m, dx, glx.DeviceArray(b), max_iter=5000, eps=1e-10)
     r = b - orc.apply(op, dx.download(), links, m, lx, ly)
     nb = np.linalg.norm(b)
     # (BiCGStab's iterated residual may drift from the true one)
@@ -196,7 +207,8 @@ def test_multishift_matches_oracle(glx, orc, lx, ly, n_shift, freq):
     kw = dict(links=links, mass=m, lx=lx, ly=ly, resid_freq_check=freq, max_iter=5000, eps=1e-10)
     X, io, _, _ = orc.cg_m("staggered_normal", b, shifts, **kw)
     xs = [glx.DeviceArray(b) for _ in shifts]  # (what they hold is overwritten)
-    ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, resid_freq_check=freq, max_iter=5000)
+    with resident_solves(glx, 1):
+        ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, resid_freq_check=freq, max_iter=5000)
     assert ig.success and abs(ig.iter - io.iter) <= freq and ig.ops_count == ig.iter + n_shift
     nb = np.linalg.norm(b)
     for k, s in enumerate(shifts):
@@ -216,7 +228,8 @@ def test_multishift_stops_at_max_iter(glx, orc):
         X, io, _, _ = orc.cg_m("staggered_normal", b, shifts, links=links, mass=m, lx=lx, ly=ly, resid_freq_check=10,
                                max_iter=stop, eps=1e-10)
         xs = [glx.DeviceArray(np.zeros_like(b)) for _ in shifts]
-        ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, max_iter=stop)
+        with resident_solves(glx, 1):
+            ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, max_iter=stop)
         assert (ig.iter, ig.success, ig.ops_count) == (io.iter, io.success, io.ops_count)
         for x, xo in zip(xs, X):
             assert relerr(x.download(), xo) < 1e-12
@@ -249,7 +262,8 @@ def gcr_both(glx, resident, h, b, x0, **kw):
     for on in (True, False):
         resident(on, 0)
         dx = glx.DeviceArray(x0)
-        info = h.solve("gcr", dx, glx.DeviceArray(b), **kw)
+        with resident_solves(glx, int(on)):
+            info = h.solve("gcr", dx, glx.DeviceArray(b), **kw)
         out.append((dx.download(), info))
     return out
 
@@ -306,7 +320,8 @@ def test_gcr_waits_that_run_out(glx, orc, resident):
     o, h, b, x0 = coarse(glx, orc, 32, 32, 8, False)
     resident(True, 1)
     dx = glx.DeviceArray(x0)
-    assert h.solve("gcr", dx, glx.DeviceArray(b), max_iter=400, eps=1e-10).success
+    with resident_solves(glx, 0, gave_up=1):
+        assert h.solve("gcr", dx, glx.DeviceArray(b), max_iter=400, eps=1e-10).success
     assert np.linalg.norm(b - orc.cstencil_apply(o, dx.download())) <= 1.01e-10 * np.linalg.norm(b)
 
 
@@ -317,23 +332,24 @@ def test_guess_stop_and_zero(glx, orc):
     kw = dict(links=links, mass=m, lx=lx, ly=ly)
     x0, _ = orc.solve("cg", "staggered_normal", b, None, max_iter=5000, eps=1e-6, **kw)
     xo, io = orc.solve("cg", "staggered_normal", b, x0, max_iter=5000, eps=1e-10, **kw)
-    dx = glx.DeviceArray(x0)
-    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
-    # (nearest: the serial sums round differently)
-    assert abs(ig.iter - io.iter) <= 1 and relerr(dx.download(), xo) < 1e-9
-    for stop in (1, 2, 7):
-        xo, io = orc.solve("cg", "staggered_normal", b, None, max_iter=stop, eps=1e-10, **kw)
+    with resident_solves(glx, 8):
+        dx = glx.DeviceArray(x0)
+        ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+        # (nearest: the serial sums round differently)
+        assert abs(ig.iter - io.iter) <= 1 and relerr(dx.download(), xo) < 1e-9
+        for stop in (1, 2, 7):
+            xo, io = orc.solve("cg", "staggered_normal", b, None, max_iter=stop, eps=1e-10, **kw)
+            dx = glx.DeviceArray(np.zeros_like(b))
+            ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=stop)
+            assert (ig.iter, ig.success, ig.ops_count) == (io.iter, io.success, io.ops_count)
+            assert relerr(dx.download(), xo) < 1e-12 and abs(ig.resSq - io.resSq) < 1e-10 * io.resSq
+            dx.upload(np.zeros_like(b))
+            im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, max_iter=stop)
+            assert not im.success and im.iter == stop and relerr(dx.download(), xo) < 1e-4
+        z = glx.DeviceArray(np.zeros_like(b))
         dx = glx.DeviceArray(np.zeros_like(b))
-        ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=stop)
-        assert (ig.iter, ig.success, ig.ops_count) == (io.iter, io.success, io.ops_count)
-        assert relerr(dx.download(), xo) < 1e-12 and abs(ig.resSq - io.resSq) < 1e-10 * io.resSq
-        dx.upload(np.zeros_like(b))
-        im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db, max_iter=stop)
-        assert not im.success and im.iter == stop and relerr(dx.download(), xo) < 1e-4
-    z = glx.DeviceArray(np.zeros_like(b))
-    dx = glx.DeviceArray(np.zeros_like(b))
-    im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, z)
-    assert im.success and im.resSq == 0.0 and not dx.download().any()
+        im = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, z)
+        assert im.success and im.resSq == 0.0 and not dx.download().any()
 
 
 def test_waits_that_run_out(glx, orc, resident):
@@ -344,10 +360,12 @@ def test_waits_that_run_out(glx, orc, resident):
     xo, io = orc.solve("cg", "staggered_normal", b, None, links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-10)
     resident(True, 1)
     dx = glx.DeviceArray(np.zeros_like(b))
-    ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
+    with resident_solves(glx, 0, gave_up=1):
+        ig = glx.dev_solve("cg", lat, "staggered_normal", m, dx, db, max_iter=5000)
     assert abs(ig.iter - io.iter) <= 1 and relerr(dx.download(), xo) < 1e-9
     dx.upload(np.zeros_like(b))
-    assert glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db).success
+    with resident_solves(glx, 0, gave_up=1):
+        assert glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db).success
     assert relerr(dx.download(), xo) < 1e-9
 
 
@@ -370,9 +388,10 @@ def test_threads_share_the_chip(glx, orc):
             got[k] = dx.download()
 
     ts = [threading.Thread(target=run, args=(k,)) for k in range(len(work))]
-    for t in ts:
-        t.start()
-    for t in ts:
-        t.join()
+    with resident_solves(glx, 3 * len(work)):
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
     for a, g in zip(alone, got):
         assert np.array_equal(a, g)
