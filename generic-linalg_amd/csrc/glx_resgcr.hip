@@ -39,8 +39,10 @@ void launch(hipStream_t st, RsGcr& g) {
   constexpr int one = int(sizeof(c128)) * 64 * M;
   g.held = std::max(0, std::min(kRgDirs, (kLds - lds) / one));
   lds += g.held * one;
+  // (the most it may ever be, the same for every solve: the attribute is the
+  // function's, and solves of other threads set it too)
   GLX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rs_gcr<M>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lds));
+                              kLds));
   hipLaunchKernelGGL(k_rs_gcr<M>, dim3(g.nblk), dim3(kRsThreads), lds, st, g);
   GLX_CHECK_LAUNCH();
 }

@@ -316,6 +316,37 @@ def test_gcr_over_several_launches(glx, orc, resident):
     assert i.success and i.iter > 520
 
 
+def test_gcr_from_several_threads(glx, orc):
+    """Solves of one kernel instance with different amounts of LDS (stencils
+    of 5 and 13 terms and several colours), from several threads at once: the
+    bits each gives alone."""
+    work = [coarse(glx, orc, *s)[1:] for s in ((32, 32, 8, False), (24, 24, 6, True), (20, 24, 4, False), (9, 7, 12, True))]
+    alone, got = [], [None] * len(work)
+    for h, b, x0 in work:
+        dx = glx.DeviceArray(x0)
+        assert h.solve("gcr", dx, glx.DeviceArray(b), max_iter=400, eps=1e-10).success
+        alone.append(dx.download())
+
+    def run(k):
+        h, b, x0 = work[k]
+        db = glx.DeviceArray(b)
+        for _ in range(40):
+            dx = glx.DeviceArray(x0)
+            h.solve("gcr", dx, db, max_iter=400, eps=1e-10)
+            x = dx.download()
+            if got[k] is None or np.array_equal(got[k], alone[k]):  # (the first that differs stays)
+                got[k] = x
+
+    ts = [threading.Thread(target=run, args=(k,)) for k in range(len(work))]
+    with resident_solves(glx, 40 * len(work)):
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    for a, g in zip(alone, got):
+        assert np.array_equal(a, g)
+
+
 def test_gcr_waits_that_run_out(glx, orc, resident):
     o, h, b, x0 = coarse(glx, orc, 32, 32, 8, False)
     resident(True, 1)
