@@ -1400,7 +1400,7 @@ int glx_set_sstep_rows(int lx, int ly, int rows) {
   return guarded([&] {
     if (lx <= 0 || ly <= 0) throw ArgError("bad lattice size");
     if (rows > 0 && (rows < 8 || rows % 4 != 0)) throw ArgError("rows must be -1, 0 or a multiple of 4 >= 8");
-    set_sstep_rows(lx, ly, rows < 0 ? -1 : rows);
+    set_sstep_rows(lx, ly, rows < 0 ? -1 : rows, true);
   });
 }
 int glx_set_sstep_form(int form, int band_rows) {
@@ -1415,7 +1415,7 @@ int glx_get_sstep_form(int* form) {
 int glx_set_sstep_form_entry(int lx, int ly, int form) {
   return guarded([&] {
     if (lx <= 0 || ly <= 0) throw ArgError("bad lattice size");
-    set_sstep_form_entry(lx, ly, form);
+    set_sstep_form_entry(lx, ly, form, true);
   });
 }
 int glx_get_sstep_form_for(int lx, int ly, int* form) {
@@ -1677,8 +1677,8 @@ int glx_autotune_sstep(glx_lattice lat, int reps, int* rows, double* ms_per_iter
     mo.link_prec = LINKS_F32;
     mo.sstep = 2;
     const int forced = sstep_rows();
-    const int saved = sstep_rows_entry(o.lx, o.ly);  // -1: none (erased again on error)
-    const int forced_form = sstep_form(), saved_form = sstep_form_entry(o.lx, o.ly);
+    const SstepEntries saved = sstep_entries(o.lx, o.ly);  // (back again on error)
+    const int forced_form = sstep_form();
     set_sstep(sstep_default(), 0);  // the tables decide while timing
     set_sstep_form(-1, 0);
     int best = 0, best_form = 0;
@@ -1698,8 +1698,7 @@ int glx_autotune_sstep(glx_lattice lat, int reps, int* rows, double* ms_per_iter
       }
       if (cand.size() > 1) cand.push_back({sstep_rows_auto(o.lx, o.ly), 1});
       for (auto [c, f] : cand) {
-        set_sstep_rows(o.lx, o.ly, c);
-        set_sstep_form_entry(o.lx, o.ly, f);
+        set_sstep_entries(o.lx, o.ly, {c, f, false, false});
         auto time_one = [&]() {
           GLX_HIP(hipMemset(x.get(), 0, size_t(n) * sizeof(c128)));
           GLX_HIP(hipDeviceSynchronize());
@@ -1718,13 +1717,11 @@ int glx_autotune_sstep(glx_lattice lat, int reps, int* rows, double* ms_per_iter
       }
     } catch (...) {
       restore();
-      set_sstep_rows(o.lx, o.ly, saved);
-      set_sstep_form_entry(o.lx, o.ly, saved_form);
+      set_sstep_entries(o.lx, o.ly, saved);
       throw;
     }
     restore();
-    set_sstep_rows(o.lx, o.ly, best);
-    set_sstep_form_entry(o.lx, o.ly, best_form);
+    set_sstep_entries(o.lx, o.ly, {best, best_form, false, false});
     if (rows) *rows = best;
     if (ms_per_iteration) *ms_per_iteration = best_ms;
   });

@@ -107,9 +107,8 @@ int sstep_default();
 int sstep_rows();
 // Per lattice size: rows per block of the s-step kernel, or 0 for the
 // one-iteration form at that size (rows < 0 removes the entry).
-void set_sstep_rows(int lx, int ly, int rows);
+void set_sstep_rows(int lx, int ly, int rows, bool by_hand);
 int sstep_rows_for(int lx, int ly);
-int sstep_rows_entry(int lx, int ly);  // the size's table entry, or -1 when it has none
 int sstep_rows_auto(int lx, int ly);
 // The form of the s-step launch on the full-lattice D^dag D: 0 blocks of four
 // waves marching a strip together through LDS rings, 1 every wave marching a
@@ -118,8 +117,16 @@ int sstep_rows_auto(int lx, int ly);
 // autotuner), else by size (sstep_form_for).
 void set_sstep_form(int form, int band_rows);
 int sstep_form();
-void set_sstep_form_entry(int lx, int ly, int form);  // -1 removes the entry
-int sstep_form_entry(int lx, int ly);                 // -1: none
+void set_sstep_form_entry(int lx, int ly, int form, bool by_hand);  // -1 removes the entry
+// The size's entries (-1: none) and whether they were set by hand, in which
+// case mixed solves of the size take that launch form instead of running
+// resident; the autotuner's (by_hand false) shape launches only.
+struct SstepEntries {
+  int rows, form;
+  bool rows_by_hand, form_by_hand;
+};
+SstepEntries sstep_entries(int lx, int ly);
+void set_sstep_entries(int lx, int ly, const SstepEntries& e);
 int sstep_form_for(int lx, int ly);
 int sw_rows_for(int lx, int ly);
 double time_sscg_traffic_impl(const DevOperator& o, int link_prec, int reps);

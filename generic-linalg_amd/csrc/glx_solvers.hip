@@ -2083,12 +2083,28 @@ SolveResult fastcg_impl(const DevOperator& o, TD* x, const TD* b, const SolveOpt
 namespace {
 std::atomic<int> g_sstep{2};
 std::atomic<int> g_sstep_rows{0};  // 0: per lattice size
-struct SsTable {
+// Choices by lattice size, installed by hand or by the autotuner.
+struct SizeTable {
+  struct Entry {
+    int v;
+    bool by_hand;
+  };
   std::mutex mu;
-  std::map<std::pair<int, int>, int> rows;
+  std::map<std::pair<int, int>, Entry> of;
+
+  void set(int lx, int ly, int v, bool by_hand) {  // v < 0: removes the entry
+    std::lock_guard<std::mutex> g(mu);
+    if (v < 0) of.erase(std::make_pair(lx, ly));
+    else of[std::make_pair(lx, ly)] = Entry{v, by_hand};
+  }
+  Entry get(int lx, int ly) {  // v = -1: none
+    std::lock_guard<std::mutex> g(mu);
+    auto it = of.find(std::make_pair(lx, ly));
+    return it != of.end() ? it->second : Entry{-1, false};
+  }
 };
-SsTable& ss_table() {
-  static SsTable t;
+SizeTable& ss_table() {
+  static SizeTable t;
   return t;
 }
 }  // namespace
@@ -2103,12 +2119,8 @@ int sstep_rows() { return g_sstep_rows.load(); }
 namespace {
 std::atomic<int> g_sstep_form{-1};  // -1: by lattice size
 std::atomic<int> g_sw_rows{0};      // 0: by lattice size
-struct FormTable {
-  std::mutex mu;
-  std::map<std::pair<int, int>, int> form;
-};
-FormTable& form_table() {
-  static FormTable t;
+SizeTable& form_table() {
+  static SizeTable t;
   return t;
 }
 }  // namespace
@@ -2121,18 +2133,9 @@ void set_sstep_form(int form, int band_rows) {
   g_sw_rows.store(band_rows);
 }
 int sstep_form() { return g_sstep_form.load(); }
-void set_sstep_form_entry(int lx, int ly, int form) {
+void set_sstep_form_entry(int lx, int ly, int form, bool by_hand) {
   if (form < -1 || form > 1) throw ArgError("s-step form entry must be -1 (remove), 0 or 1");
-  FormTable& t = form_table();
-  std::lock_guard<std::mutex> g(t.mu);
-  if (form < 0) t.form.erase(std::make_pair(lx, ly));
-  else t.form[std::make_pair(lx, ly)] = form;
-}
-int sstep_form_entry(int lx, int ly) {
-  FormTable& t = form_table();
-  std::lock_guard<std::mutex> g(t.mu);
-  auto it = t.form.find(std::make_pair(lx, ly));
-  return it != t.form.end() ? it->second : -1;
+  form_table().set(lx, ly, form, by_hand);
 }
 // The form a solve of an lx x ly D^dag D takes: the process-wide choice if
 // one is set, else the size's entry, else the wave strips where the lattice
@@ -2144,7 +2147,7 @@ int sstep_form_entry(int lx, int ly) {
 int sstep_form_for(int lx, int ly) {
   const int f = g_sstep_form.load();
   if (f >= 0) return f;
-  const int e = sstep_form_entry(lx, ly);
+  const int e = form_table().get(lx, ly).v;
   if (e >= 0) return e;
   const long nstrip = (lx + kSwOwn - 1) / kSwOwn;
   const long waves = nstrip * ((ly + 51) / 52);
@@ -2164,11 +2167,22 @@ int sw_rows_for(int lx, int ly) {
   while (rows < need && rows + 6 <= kSwMaxRows) rows += 6;
   return rows;
 }
-void set_sstep_rows(int lx, int ly, int rows) {
-  SsTable& t = ss_table();
-  std::lock_guard<std::mutex> g(t.mu);
-  if (rows < 0) t.rows.erase(std::make_pair(lx, ly));
-  else t.rows[std::make_pair(lx, ly)] = rows;
+void set_sstep_rows(int lx, int ly, int rows, bool by_hand) { ss_table().set(lx, ly, rows, by_hand); }
+SstepEntries sstep_entries(int lx, int ly) {
+  const SizeTable::Entry r = ss_table().get(lx, ly), f = form_table().get(lx, ly);
+  return {r.v, f.v, r.by_hand, f.by_hand};
+}
+void set_sstep_entries(int lx, int ly, const SstepEntries& e) {
+  ss_table().set(lx, ly, e.rows, e.rows_by_hand);
+  form_table().set(lx, ly, e.form, e.form_by_hand);
+}
+// Whether the caller has chosen how mixed solves of this size are launched: by
+// the process-wide settings or by an entry for the size.  (An entry of the
+// autotuner's is the fastest of the launch forms, not a choice against the
+// resident one.)
+static bool sstep_chosen(int lx, int ly) {
+  const SstepEntries e = sstep_entries(lx, ly);
+  return sstep_default() != 2 || sstep_rows() != 0 || sstep_form() >= 0 || e.rows_by_hand || e.form_by_hand;
 }
 // Without a table entry: the fewest rows per block (8, 16, 32, 64, 128) that
 // keep the grid within 512 blocks, two per CU, else 256 (measured: 256^2 and
@@ -2181,19 +2195,11 @@ int sstep_rows_auto(int lx, int ly) {
     if (strips * ((ly + r - 1) / r) <= 512) return r;
   return 256;
 }
-int sstep_rows_entry(int lx, int ly) {
-  SsTable& t = ss_table();
-  std::lock_guard<std::mutex> g(t.mu);
-  auto it = t.rows.find(std::make_pair(lx, ly));
-  return it != t.rows.end() ? it->second : -1;
-}
 int sstep_rows_for(int lx, int ly) {
   const int forced = g_sstep_rows.load();
   if (forced > 0) return forced;
-  SsTable& t = ss_table();
-  std::lock_guard<std::mutex> g(t.mu);
-  auto it = t.rows.find(std::make_pair(lx, ly));
-  return it != t.rows.end() ? it->second : sstep_rows_auto(lx, ly);
+  const int e = ss_table().get(lx, ly).v;
+  return e >= 0 ? e : sstep_rows_auto(lx, ly);
 }
 
 // Columns per lane of the s-step kernel: D^dag D in strips of 128 columns
@@ -2802,8 +2808,8 @@ SolveResult dev_cg_m(const DevOperator& op, void* const* xs, const void* b, int 
                          resid_freq_check, worst_first, o);
 }
 SolveResult dev_cg_mixed(const DevOperator& op, void* x, const void* b, const SolveOpts& o, const MixedOpts& m) {
-  // resident where the system fits, unless a launch form was asked for
-  if (m.sstep == 0 && sstep_default() == 2 && sstep_rows() == 0 && sstep_form() < 0)
+  // resident where the system fits, unless a launch form was chosen
+  if (m.sstep == 0 && !sstep_chosen(op.lx, op.ly))
     if (auto r = rs_solve(op, x, b, o, RSF_MIXED, m)) return *r;
   if (!real_op(op) && (m.sstep ? m.sstep : sstep_default()) == 2 && sscg_fits(op)) {
     const int rows = sstep_rows_for(op.lx, op.ly);  // 0: the one-iteration form for this size

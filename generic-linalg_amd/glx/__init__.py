@@ -684,7 +684,9 @@ def set_sstep(s: int = 2, rows: int = 0):
 
 
 def set_sstep_rows(lx: int, ly: int, rows: int):
-    """Per-size entry: s-step rows per block, 0 = one-iteration form, -1 = remove."""
+    """Per-size entry: s-step rows per block, 0 = one-iteration form, -1 =
+    remove.  Mixed solves of a size with an entry run in launches, also where
+    they would run resident."""
     _check(lib().glx_set_sstep_rows(lx, ly, rows), "glx_set_sstep_rows")
 
 
@@ -703,7 +705,8 @@ def get_sstep_form() -> int:
 
 
 def set_sstep_form_entry(lx: int, ly: int, form: int):
-    """Per-size entry of the s-step form (0 or 1), -1 = remove."""
+    """Per-size entry of the s-step form (0 or 1), -1 = remove; like
+    set_sstep_rows it keeps mixed solves of the size in launches."""
     _check(lib().glx_set_sstep_form_entry(lx, ly, form), "glx_set_sstep_form_entry")
 
 

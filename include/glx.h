@@ -440,7 +440,8 @@ int glx_dev_eo_reconstruct(glx_lattice lat, double mass, double* x_dev, const do
 /* Launch tuning of the single-pass CG and the mixed-precision CG: iterations
  * per enqueued group (default 16; rounded up to even where the iteration is
  * self-finalising) and whether a group is captured once as a hipGraph and
- * replayed (default 0: measured slightly slower than direct launches). */
+ * replayed (default 0: measured slightly slower than direct launches).  A
+ * solve that runs resident (below) has no groups. */
 int glx_set_tuning(int group, int use_graph);
 /* Resident solves (no reference counterpart): where a system fits the chip's
  * registers, one launch keeps it there and runs the whole solve (CG on D^dag D
@@ -453,8 +454,12 @@ int glx_set_tuning(int group, int use_graph);
  * spins: how often a block polls for another block's value before the launch
  * gives up and the solve is repeated with a launch per iteration (0: the
  * default, about a second).  A launch form chosen by glx_set_sstep or
- * glx_set_sstep_form (other than their defaults) keeps the mixed solver on
- * that form. */
+ * glx_set_sstep_form (other than their defaults), or for a size by
+ * glx_set_sstep_rows or glx_set_sstep_form_entry, keeps the mixed solver on
+ * that form; an entry that glx_autotune_sstep installs does not (it compares
+ * launch forms).  Settings that only shape launches -- glx_set_tuning,
+ * glx_set_normal_rows and the autotuners' entries -- apply to the solves that
+ * run in launches. */
 int glx_set_resident(int on, int spins);
 /* How many solves of this process ran resident so far, and how many had a
  * resident launch that gave up and were repeated with a launch per iteration
@@ -473,7 +478,9 @@ int glx_set_sstep(int s, int rows);
 int glx_get_sstep(int* s, int* rows);
 /* The per-size table: rows per block of the s-step kernel for an lx x ly
  * lattice, or 0 = the one-iteration form at that size; -1 removes the entry.
- * glx_get_sstep_rows returns what a solve of that size would use. */
+ * Mixed solves of a size with an entry run in launches also where they fit
+ * the chip (glx_set_resident), unless the autotuner installed it.
+ * glx_get_sstep_rows returns what a solve of that size in launches uses. */
 int glx_set_sstep_rows(int lx, int ly, int rows);
 int glx_get_sstep_rows(int lx, int ly, int* rows);
 /* The form of the s-step launch on the full-lattice D^dag D (no reference
@@ -484,8 +491,9 @@ int glx_get_sstep_rows(int lx, int ly, int* rows);
  * 52 that keep the launch within 1024 waves; at most 56).  form -1 (default)
  * chooses per lattice size: the size's entry (glx_set_sstep_form_entry, set
  * by glx_autotune_sstep), else form 1 from 512^2 sites up to lattices that
- * fit 1024 waves at bands of 52 rows, form 0 otherwise.
- * glx_get_sstep_form_for returns what a solve of that size would use.  The
+ * fit 1024 waves at bands of 52 rows, form 0 otherwise.  An entry set by
+ * hand keeps mixed solves of its size in launches, as for the rows.
+ * glx_get_sstep_form_for returns what a solve of that size in launches uses.  The
  * mixed CG of the even/odd solve (the compact Schur operator) follows the
  * same choice, except that by size it takes form 1 only above 512^2 sites. */
 int glx_set_sstep_form(int form, int band_rows);
@@ -509,7 +517,7 @@ int glx_autotune_sstep(glx_lattice lat, int reps, int* rows, double* ms_per_iter
  * grid within 512 blocks (64 lanes of 1 FP64 or 2 FP32 sites per block row;
  * compact rows of lx / 2 sites for the even/odd Schur operator), else 256.
  * rows = -1 with a size removes that size's entry.
- * glx_get_normal_rows returns what a solve of that size would use (for
+ * glx_get_normal_rows returns what a solve of that size in launches uses (for
  * lx = ly = 0, the default itself).
  * The row-marching kernel needs lx % 64 == 0 (FP64) or lx % 128 == 0 (FP32,
  * two sites per lane), ly % 4 == 0, ly >= 8; other sizes always use the

@@ -383,6 +383,53 @@ def test_guess_stop_and_zero(glx, orc):
         assert im.success and im.resSq == 0.0 and not dx.download().any()
 
 
+def test_a_chosen_launch_form_is_taken(glx, orc):
+    """A launch form set for the process or for the lattice's size keeps the
+    mixed solve, even/odd included, in launches; another size's entry, the
+    autotuner's and a removed one do not."""
+    lx, ly, m = 256, 64, 0.1
+    links, b, lat, db = system(glx, orc, lx, ly)
+
+    def solves(n):
+        for _ in range(2):
+            dx = glx.DeviceArray(np.zeros_like(b))
+            with resident_solves(glx, n):
+                info = glx.dev_cg_mixed(lat, "staggered_normal", m, dx, db)
+            r = b - orc.apply("staggered_normal", dx.download(), links, m, lx, ly)
+            assert info.success and np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(b)
+        with resident_solves(glx, n):
+            assert glx.dev_solve_staggered_eo(lat, m, glx.DeviceArray(np.zeros_like(b)), db, "mixed")[0].success
+
+    solves(1)
+    try:
+        for rows in (0, 8, 16):
+            glx.set_sstep_rows(lx, ly, rows)
+            solves(0)
+        glx.set_sstep_rows(lx, ly, -1)
+        for form in (0, 1):
+            glx.set_sstep_form_entry(lx, ly, form)
+            solves(0)
+        glx.set_sstep_form_entry(lx, ly, -1)
+        glx.set_sstep_rows(lx, 2 * ly, 8)
+        solves(1)
+        glx.set_sstep_rows(lx, ly, 8)
+        glx.autotune_sstep(lat, reps=4)  # (replaces the entry)
+        solves(1)
+        glx.set_sstep_rows(lx, ly, 8)
+        solves(0)
+    finally:
+        glx.set_sstep_rows(lx, ly, -1)
+        glx.set_sstep_rows(lx, 2 * ly, -1)
+        glx.set_sstep_form_entry(lx, ly, -1)
+    solves(1)
+    for s, rows in ((1, 0), (2, 8)):
+        glx.set_sstep(s, rows)
+        try:
+            solves(0)
+        finally:
+            glx.set_sstep()
+
+
 def test_waits_that_run_out(glx, orc, resident):
     """With a single poll per wait the launch gives up, and the solve runs with
     a launch per iteration: the same answer."""
