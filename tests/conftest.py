@@ -43,6 +43,19 @@ def resident(glx):
 
 
 @pytest.fixture
+def in_launches(resident):
+    """Solves run in launches, also where their system fits the chip."""
+    resident(False)
+
+
+@pytest.fixture(params=[True, False], ids=["resident", "launches"])
+def runs_resident(request, resident):
+    """Once with solves resident where their system fits, once in launches."""
+    resident(request.param)
+    return request.param
+
+
+@pytest.fixture
 def rows_reset(glx, monkeypatch):
     """Launch-shape table entries a test sets through glx.set_normal_rows are
     removed afterwards and the default goes back to -1 (by block count), so

@@ -22,8 +22,8 @@ the serial sums alone move the reference's solution by 5e-12 (256^2) and
   staggered 1024^2, m = 0.02, theta ~ N(0, 0.5^2) (beta = 4):
       FP64 CG (reference order) with the oracle's iterations and x within
       1e-12 of the correctly reduced oracle's; single-pass FP64 CG; the
-      mixed-precision CG in both forms (two iterations per launch and one)
-      with FP32 and FP16 links, each with its true residual recomputed by
+      mixed-precision CG in its three forms (resident, two iterations per
+      launch and one) with FP32 and FP16 links, each with its true residual recomputed by
       the oracle's FP64 operator and its error against the oracle's FP64
       solution printed and bounded.
   multishift batch: one lattice for each L in {64, 128, 192, 256, 384, 512},
@@ -71,7 +71,7 @@ def check_fp64_cg(what, xg, ig, serial, extended, tol=1e-12):
     assert d_gs <= d_se + tol, (d_gs, d_se)
 
 
-def test_c2_cg_normal_matches_oracle(glx, orc, c2):
+def test_c2_cg_normal_matches_oracle(glx, orc, runs_resident, c2):
     links, b = c2
     kw = dict(links=links, mass=M2, lx=L2, ly=L2, max_iter=100000, eps=1e-10)
     serial, extended = oracle_pair(orc, "cg", "staggered_normal", b, kw)
@@ -83,7 +83,7 @@ def test_c2_cg_normal_matches_oracle(glx, orc, c2):
     assert abs(ig.resSq - io.resSq) <= 0.05 * io.resSq
 
 
-def test_c2_bicgstab_inside_oracle_envelope(glx, orc, c2):
+def test_c2_bicgstab_inside_oracle_envelope(glx, orc, runs_resident, c2):
     links, b = c2
     kw = dict(links=links, mass=M2, lx=L2, ly=L2, max_iter=100000, eps=1e-10)
     x0, i0, its, dx = bicgstab_envelope(orc, "staggered", b, kw)
@@ -109,12 +109,33 @@ def c3(glx, orc):
     return links, bc, serial[0], serial[1], lat, serial, extended
 
 
+@pytest.fixture(scope="module")
+def c3_at(orc, c3):
+    """The oracle's solves of the 1024^2 system: (history to max_iter
+    iterations, the pair stopped at max_iter), each computed once."""
+    links, b = c3[:2]
+    kw = dict(links=links, mass=M3, lx=L3, ly=L3, eps=1e-10)
+    hist, pair = {}, {}
+
+    def history(n):
+        if n not in hist:
+            hist[n] = orc.solve("cg", "staggered_normal", b, None, hist=True, max_iter=n, **kw)[2]
+        return hist[n]
+
+    def stopped(n):
+        if n not in pair:
+            pair[n] = oracle_pair(orc, "cg", "staggered_normal", b, dict(kw, max_iter=n))
+        return pair[n]
+
+    return history, stopped
+
+
 def _true_relres(orc, links, b, x):
     r = b - orc.apply("staggered_normal", x, links, M3, L3, L3)
     return float(np.linalg.norm(r) / np.linalg.norm(b))
 
 
-def test_c3_fp64_cg_matches_oracle(glx, orc, c3):
+def test_c3_fp64_cg_matches_oracle(glx, runs_resident, c3, c3_at):
     """At cond(A) ~ 1e4 the iterated residual of any FP64 CG is fixed only to
     ~1 % by rounding, so the stop (relres < 1e-10) of two valid
     implementations may fall one iteration apart where the residual is within
@@ -126,18 +147,16 @@ def test_c3_fp64_cg_matches_oracle(glx, orc, c3):
     assert ig.success and ig.ops_count == ig.iter + 2
     if ig.iter != io.iter:
         assert abs(ig.iter - io.iter) == 1, (ig.iter, io.iter)
-        _, io_h, hist = orc.solve("cg", "staggered_normal", b, None, hist=True, **dict(kw, max_iter=max(ig.iter,
-                                                                                                   io.iter)))
+        hist = c3_at[0](max(ig.iter, io.iter))
         k = min(ig.iter, io.iter) - 1  # the oracle's relres where the two stops differ
         assert abs(hist[k] - 1e-10) <= 0.03e-10, hist[k]
-        serial, extended = pmap(lambda red: orc.solve("cg", "staggered_normal", b, None, reductions=red,
-                                                      **dict(kw, max_iter=ig.iter)), ["serial", "extended"])
+        serial, extended = c3_at[1](ig.iter)
         print(f"C3: stops one iteration apart (oracle relres {hist[k]:.4e} at iteration {k + 1}); compared after "
               f"{ig.iter} iterations")
     check_fp64_cg("C3 FP64 CG", xg, ig, serial, extended)
 
 
-def test_c3_fp64_single_pass_cg(glx, orc, c3):
+def test_c3_fp64_single_pass_cg(glx, orc, runs_resident, c3):
     links, b, xo, io, lat, _, extended = c3
     dx = glx.DeviceArray(np.zeros_like(b))
     info = glx.dev_cg_fused(lat, "staggered_normal", M3, dx, glx.DeviceArray(b), max_iter=100000, eps=1e-10)
@@ -150,15 +169,16 @@ def test_c3_fp64_single_pass_cg(glx, orc, c3):
     assert relerr(x, xo) <= 1e-11
 
 
-@pytest.mark.parametrize("sstep", [2, 1])
+@pytest.mark.parametrize("sstep,on", [(2, True), (2, False), (1, True)], ids=["resident", "sstep", "one_iteration"])
 @pytest.mark.parametrize("link_prec", [1, 2])
-def test_c3_mixed_against_oracle(glx, orc, c3, sstep, link_prec):
+def test_c3_mixed_against_oracle(glx, orc, resident, c3, sstep, on, link_prec):
     """Mixed precision (FP32 bulk, FP32 or FP16 links, FP64 reliable updates
     at delta 0.1): the oracle's FP64 operator recomputes the true residual of
     the returned x (<= 1e-10, equal to the one the solver reports), and x is
     within 5e-11 of the oracle's FP64 solution (measured 5e-12: both
     solutions carry residuals of 1e-10 whose error components differ)."""
     links, b, xo, io, lat, _, _ = c3
+    resident(on)
     glx.set_sstep(sstep)
     try:
         dx = glx.DeviceArray(np.zeros_like(b))

@@ -75,7 +75,7 @@ def test_prepare_reconstruct(glx, orc):
 
 
 @pytest.mark.parametrize("lx,ly,m", [(128, 64, 0.1), (256, 128, 0.05)])
-def test_eo_solve_matches_oracle_pipeline(glx, orc, lx, ly, m):
+def test_eo_solve_matches_oracle_pipeline(glx, orc, runs_resident, lx, ly, m):
     links, bc, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=21 + lx)
     kw = dict(links=links, mass=m, lx=lx, ly=ly, max_iter=5000, eps=1e-10)
     be = orc.eoprec_prepare(bc, links, m, lx, ly)
@@ -101,7 +101,7 @@ def test_eo_solve_matches_oracle_pipeline(glx, orc, lx, ly, m):
 
 
 @pytest.mark.parametrize("method", ["cg_fused", "mixed", "mixed_f16"])
-def test_eo_solve_fast_methods(glx, orc, method):
+def test_eo_solve_fast_methods(glx, orc, runs_resident, method):
     lx, ly, m = 256, 64, 0.05
     links, bc, _ = lattice_inputs(orc, lx, ly, beta=6.25, seed=31)
     lat = glx.Lattice(links, lx, ly)

@@ -6,14 +6,15 @@ solve stops on it.  Checks: the returned FP64 true relative residual is
 <= tol; the solution is within ENVELOPE times the error of the oracle's FP64
 CG solve at the same tolerance, both measured against the oracle's solve at
 1e-13 (helpers.cg_envelope); the device's reported residual equals the
-oracle's recomputation.
+oracle's recomputation.  Every test runs twice: resident where the system
+fits the chip, and in launches.
 """
 import numpy as np
 import pytest
 
 from helpers import ENVELOPE, cg_envelope, lattice_inputs, relerr
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("runs_resident")]
 
 
 @pytest.mark.parametrize("link_prec", [1, 2])

@@ -53,7 +53,7 @@ def test_normal_fp32_matches_tiled(glx, orc, rows_reset, lx, ly, rows, link_prec
 
 
 @pytest.mark.parametrize("rows", [0, 8, 16])
-def test_cg_with_normal_kernel(glx, orc, rows_reset, rows):
+def test_cg_with_normal_kernel(glx, orc, rows_reset, in_launches, rows):
     """The reference-order CG keeps exact iteration and ops counts with the
     row-marching kernel in the loop (its reductions are FP64 and the stencil
     agrees with the oracle to rounding)."""
@@ -71,7 +71,7 @@ def test_cg_with_normal_kernel(glx, orc, rows_reset, rows):
 
 
 @pytest.mark.parametrize("rows", [8, 16, 32])
-def test_mixed_and_fused_with_normal_kernel(glx, orc, rows_reset, rows):
+def test_mixed_and_fused_with_normal_kernel(glx, orc, rows_reset, in_launches, rows):
     lx = ly = 128
     mass = 0.05
     links, bc, _ = lattice_inputs(orc, lx, ly, beta=4.0, seed=78)

@@ -198,7 +198,7 @@ def test_laplacians_on_a_lattice_with_links(glx, orc, solver, op):
 
 @pytest.mark.parametrize("lx,ly,n_shift,freq", [(4, 8, 1, 1), (4, 8, 16, 10), (60, 9, 5, 3), (61, 23, 16, 10),
                                                 (130, 70, 2, 7), (200, 144, 12, 10)])
-def test_multishift_matches_oracle(glx, orc, lx, ly, n_shift, freq):
+def test_multishift_matches_oracle(glx, orc, runs_resident, lx, ly, n_shift, freq):
     """Every shift's solution and residual, and the iterations (a check apart
     where a shift crosses the tolerance within rounding)."""
     m = 0.1
@@ -207,7 +207,7 @@ def test_multishift_matches_oracle(glx, orc, lx, ly, n_shift, freq):
     kw = dict(links=links, mass=m, lx=lx, ly=ly, resid_freq_check=freq, max_iter=5000, eps=1e-10)
     X, io, _, _ = orc.cg_m("staggered_normal", b, shifts, **kw)
     xs = [glx.DeviceArray(b) for _ in shifts]  # (what they hold is overwritten)
-    with resident_solves(glx, 1):
+    with resident_solves(glx, int(runs_resident)):
         ig = glx.dev_cg_m(lat, "staggered_normal", m, xs, db, shifts, resid_freq_check=freq, max_iter=5000)
     assert ig.success and abs(ig.iter - io.iter) <= freq and ig.ops_count == ig.iter + n_shift
     nb = np.linalg.norm(b)

@@ -79,7 +79,7 @@ def test_wide_eo_schur_fp64(glx, orc, rows_reset, inputs, rows):
 
 
 @pytest.mark.parametrize("rows", WIDE)
-def test_wide_single_pass_cg(glx, orc, rows_reset, inputs, rows):
+def test_wide_single_pass_cg(glx, orc, rows_reset, in_launches, inputs, rows):
     links, bc = inputs
     m = 0.05
     glx.set_normal_rows(LX, LY, 16, rows)

@@ -16,6 +16,10 @@ The squared true residual resSq is a 1e-20-level quantity formed from the
 solution; it is compared through the solution and by being below eps^2 |b|^2
 whenever the solve reports success.  Verbosity lines must agree in every
 field except the last digits of residuals.
+
+Every test runs twice: resident where the system fits the chip, and in
+launches, which also serve the larger systems and every resident launch that
+gave up.
 """
 import numpy as np
 import pytest
@@ -23,7 +27,7 @@ import pytest
 from helpers import (bicgstab_envelope, check_in_envelope, lattice_inputs, oracle_text_envelope, perturbed, pmap,
                      relerr, text_envelope)
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("runs_resident")]
 
 def xtol(op):
     return 1e-13 if op.startswith("laplace") else 1e-11

@@ -15,13 +15,15 @@ true residual as in the one-iteration form.  Checks per case:
   * max_iter stops at odd and even counts, frequent reliable updates
     (delta = 0.5), a nonzero initial guess, b = 0, graph replay and other
     rows per block.
+Systems of these sizes would run resident (test_gpu_resident.py); here they
+run in launches.
 """
 import numpy as np
 import pytest
 
 from helpers import ENVELOPE, cg_envelope, eo_envelope, lattice_inputs, relerr
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("in_launches")]
 
 
 def _solve(glx, lat, mass, b, x0=None, sstep=2, rows=0, **kw):

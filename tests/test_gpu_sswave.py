@@ -214,7 +214,7 @@ def test_wave_form_even_odd(glx, orc, lx, ly, link):
     assert abs(info.iter - i0.iter) <= max(6, 0.03 * i0.iter), (info.iter, i0.iter)
 
 
-def test_wave_form_even_odd_workload_1024(glx, orc):
+def test_wave_form_even_odd_workload_1024(glx, orc, in_launches):
     """The 1024 x 1024 even/odd solve (m = 0.02, theta ~ N(0, 0.5^2)) in the
     wave-strip form (its default at this size) against the oracle's FP64
     even/odd pipeline."""
