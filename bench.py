@@ -642,9 +642,6 @@ def main():
         tuned_ss = {"rows": args.sstep_rows}
     else:
         tuned_ss = glx.autotune_sstep(lat, reps=40)
-    # the mixed solve runs in one launch where the lattice fits 256 tiles of at
-    # most 60 x 80 sites and no launch form was asked for
-    resident = args.sstep_form is None and -(-L // 60) * -(-L // 80) <= 256
     d_b = glx.DeviceArray(b)
     d_x = glx.DeviceArray(np.zeros_like(b))
     d_x64 = glx.DeviceArray(np.zeros_like(b))
@@ -697,9 +694,11 @@ def main():
         dt, infom1 = solve_mixed(1)
         tm1.append(dt)
     tmx = []
+    ran0, gave_up0 = glx.resident_counts()
     for _ in range(args.steps):
         dt, infomx = solve_mixed()
         tmx.append(dt)
+    ran, gave_up = (n - n0 for n, n0 in zip(glx.resident_counts(), (ran0, gave_up0)))
     ms64 = float(np.median(t64)) * 1e3
     msfu = float(np.median(tfu)) * 1e3
     msmx = float(np.median(tmx)) * 1e3
@@ -785,7 +784,9 @@ def main():
         "speedup_vs_fp64": round(ms64 / msmx, 3),
         "speedup_basis": "plain FP64 GPU CG in the reference's order of operations (glx_dev_solve)",
         "speedup_vs_fp64_fused": round(msfu / msmx, 3),
-        "mixed_form": ("one launch per solve, the system in registers" if resident else
+        "mixed_resident_solves": ran,
+        "mixed_resident_gave_up": gave_up,
+        "mixed_form": ("one launch per solve, the system in registers" if ran else
                        ("s-step, two CG iterations per launch, "
                         + ("wave strips (form 1)" if glx.get_sstep_form_for(L, L) == 1
                            else f"{tuned_ss['rows']} rows per block (form 0)")

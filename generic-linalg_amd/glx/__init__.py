@@ -208,12 +208,10 @@ def lib():
         L.glx_dev_cg_fused.argtypes = [vp, i, d, vp, vp, i, d, VP, IP]
         L.glx_set_tuning.restype = i
         L.glx_set_tuning.argtypes = [i, i]
-        if hasattr(L, "glx_set_resident"):  # absent from builds that predate it
-            L.glx_set_resident.restype = i
-            L.glx_set_resident.argtypes = [i, i]
-        if hasattr(L, "glx_get_resident_counts"):
-            L.glx_get_resident_counts.restype = i
-            L.glx_get_resident_counts.argtypes = [C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
+        L.glx_set_resident.restype = i
+        L.glx_set_resident.argtypes = [i, i]
+        L.glx_get_resident_counts.restype = i
+        L.glx_get_resident_counts.argtypes = [C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]
         L.glx_set_sstep.restype = i
         L.glx_set_sstep.argtypes = [i, i]
         L.glx_get_sstep.restype = i
