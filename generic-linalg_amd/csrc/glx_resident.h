@@ -481,7 +481,7 @@ void rs_launch_cg_m(hipStream_t st, const RsGeom& g, const RsSolve& so, const Rs
 
 // The resident blocks of every solve in flight on a device, over all host
 // threads, stay within its CUs, one block each: a solve waits here until its
-// blocks fit.  Held from before the launch until the stream has drained.
+// turn has come and its blocks fit.  Held from before the launch until the stream has drained.
 class RsReserve {
  public:
   explicit RsReserve(int blocks);

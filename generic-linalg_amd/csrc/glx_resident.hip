@@ -1,11 +1,10 @@
 // glx_resident.hip -- the resident-system kernels' instances, launch shapes
 // and host-side bookkeeping (glx_resident.h).
 #include "glx_resident.h"
+#include "glx_slots.h"
 
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
-#include <mutex>
 
 namespace glx {
 
@@ -33,14 +32,9 @@ int device_cus(int dev) {
   return n;
 }
 
-struct Slots {
-  std::mutex mu;
-  std::condition_variable cv;
-  int used[kMaxDevices] = {};
-};
-Slots& slots() {
-  static Slots* s = new Slots;  // outlives every static user
-  return *s;
+FairSlots& slots(int dev) {
+  static FairSlots* s = new FairSlots[kMaxDevices];  // outlives every static user
+  return s[dev];
 }
 
 __global__ __launch_bounds__(kBlock) void k_rs_fill(unsigned long long* q, long n, RsOut* out) {
@@ -134,19 +128,8 @@ void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so) 
 }
 
 RsReserve::RsReserve(int blocks) : dev_(current_device()), blocks_(blocks) {
-  const int cap = std::max(device_cus(dev_), blocks);
-  Slots& t = slots();
-  std::unique_lock<std::mutex> l(t.mu);
-  t.cv.wait(l, [&] { return t.used[dev_] + blocks_ <= cap; });
-  t.used[dev_] += blocks_;
+  slots(dev_).acquire(blocks_, device_cus(dev_));
 }
-RsReserve::~RsReserve() {
-  Slots& t = slots();
-  {
-    std::lock_guard<std::mutex> l(t.mu);
-    t.used[dev_] -= blocks_;
-  }
-  t.cv.notify_all();
-}
+RsReserve::~RsReserve() { slots(dev_).release(blocks_); }
 
 }  // namespace glx
