@@ -480,8 +480,8 @@ bool rs_plan_one_row(int lx, int ly, int halo, RsGeom& g);
 void rs_launch_cg_m(hipStream_t st, const RsGeom& g, const RsSolve& so, const RsShiftSet& sh);
 
 // The resident blocks of every solve in flight on a device, over all host
-// threads, stay within its CUs, one block each: a solve waits here until its
-// turn has come and its blocks fit.  Held from before the launch until the stream has drained.
+// threads, stay within its CUs and each XCD's, one block each (glx_slots.h): a
+// solve waits here until its turn has come and its blocks fit.  Held from before the launch until the stream has drained.
 class RsReserve {
  public:
   explicit RsReserve(int blocks);
@@ -490,7 +490,7 @@ class RsReserve {
   RsReserve& operator=(const RsReserve&) = delete;
 
  private:
-  int dev_, blocks_;
+  int dev_, slots_;
 };
 
 }  // namespace glx

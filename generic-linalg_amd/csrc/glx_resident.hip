@@ -127,9 +127,9 @@ void rs_launch(hipStream_t st, const RsGeom& g, RsMode mode, const RsSolve& so) 
   else launch<c64, RS_MIXED>(st, g, so);
 }
 
-RsReserve::RsReserve(int blocks) : dev_(current_device()), blocks_(blocks) {
-  slots(dev_).acquire(blocks_, device_cus(dev_));
+RsReserve::RsReserve(int blocks) : dev_(current_device()), slots_(resident_slots(blocks)) {
+  slots(dev_).acquire(slots_, device_cus(dev_));
 }
-RsReserve::~RsReserve() { slots(dev_).release(blocks_); }
+RsReserve::~RsReserve() { slots(dev_).release(slots_); }
 
 }  // namespace glx

@@ -7,6 +7,15 @@
 
 namespace glx {
 
+// The slots a launch of resident blocks takes: workgroups go round the eight
+// XCDs in turn, so an XCD holds up to ceil(blocks / 8) of them.  Counted in
+// whole rounds, launches that fit the device fit every XCD; counted by blocks,
+// 65 and 190 blocks (255 of 256 CUs) could want 9 + 24 of one XCD's 32, and two
+// launches that each miss a block on another XCD would wait for each other
+// until their polls run out.
+constexpr int kXcds = 8;
+constexpr int resident_slots(int blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
+
 // A count that callers take from and give back, first come first served: one
 // that asks for much is not passed over for ever by others that fit beside
 // what is in use.

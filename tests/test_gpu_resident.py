@@ -447,6 +447,25 @@ def test_waits_that_run_out(glx, orc, resident):
     assert relerr(dx.download(), xo) < 1e-9
 
 
+def test_no_launch_waits_for_another(glx, orc):
+    """Solves of 65 and 190 blocks, which an XCD would have 9 + 24 of for its
+    32 CUs, from two threads over and over: none gives up."""
+    m = 0.1
+    work = [system(glx, orc, lx, ly) for lx, ly in ((290, 208), (600, 600))]
+
+    def run(k):
+        _, b, lat, db = work[k]
+        for _ in range(100 if k == 0 else 50):
+            glx.dev_cg_mixed(lat, "staggered_normal", m, glx.DeviceArray(np.zeros_like(b)), db)
+
+    ts = [threading.Thread(target=run, args=(k,)) for k in range(2)]
+    with resident_solves(glx, 150):
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+
+
 def test_threads_share_the_chip(glx, orc):
     """Solves from several host threads at once, together wanting more blocks
     than there are CUs, give the bits each gives alone."""

@@ -1,6 +1,7 @@
 """The reservation of resident blocks (glx_slots.h) in host threads: within
 the cap, and in the order asked for, so that a large solve gets its turn while
-small ones, which would fit beside each other, keep coming."""
+small ones, which would fit beside each other, keep coming; and launches that
+fit the device together fit each of its XCDs."""
 import os
 import subprocess
 
@@ -67,6 +68,19 @@ int main() {
     for (auto& t : ts) t.join();
     if (over != 0) return fail("beyond the cap");
     if (served != 4000 || s.used() != 0 || s.waiting() != 0) return fail("not everyone was served");
+  }
+  {
+    // two launches within 256 CUs, and three: each XCD's share within its 32
+    auto share = [](int blocks) { return (blocks + 7) / 8; };
+    for (int a = 1; a <= 256; a++)
+      for (int b = 1; b <= a; b++) {
+        const int two = glx::resident_slots(a) + glx::resident_slots(b);
+        if (two <= 256 && share(a) + share(b) > 32) return fail("two launches beyond an XCD");
+        for (int c = 1; c <= b; c++)
+          if (two + glx::resident_slots(c) <= 256 && share(a) + share(b) + share(c) > 32)
+            return fail("three launches beyond an XCD");
+      }
+    if (glx::resident_slots(256) != 256 || glx::resident_slots(1) > 256) return fail("a launch that no longer fits");
   }
   std::printf("ok\n");
   return 0;
