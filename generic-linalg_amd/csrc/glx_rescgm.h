@@ -8,7 +8,7 @@
 // the next iteration's <p, Ap> is on its way.  The shifts' recurrences are one
 // lane's each.  One row per wave (R = 1): with 16 shifts x_s and p_s take 128
 // registers of a lane, so lattices up to 256 tiles of 60 x 8 sites run here.
-// The whole solve, 200 x 144, 12 shifts, residuals included: 7.4 ms with a
+// The whole solve, 200 x 144, 12 shifts, residuals included: 7.6 ms with a
 // launch per phase, 2.1 ms here.
 #pragma once
 

@@ -20,8 +20,8 @@
 // on both sides.
 //
 // Measured (us per iteration: reference order, single-pass FP64, mixed):
-// 64^2 4.3, 2.9, 3.2; 256^2 5.3, 3.6, 3.6; 512^2 6.8, 4.6, 4.4; 1024^2 10.6,
-// 10.4, 6.1.  A launch per iteration took 17, 12, 14; 18, 12, 10; 21, 13, 10;
+// 64^2 4.1, 2.8, 2.9; 256^2 5.1, 3.5, 3.2; 512^2 6.3, 4.8, 4.0; 1024^2 10.5,
+// 10.6, 6.2.  A launch per iteration took 17, 12, 14; 18, 12, 10; 21, 13, 10;
 // 38, 30, 14.  (Of an iteration at 256^2, 1.3 us is the round trip of the
 // reduction, the rest the latencies of the hops, LDS and block sums.)
 //
